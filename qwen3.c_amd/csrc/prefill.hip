@@ -25,6 +25,7 @@
 // routing, shared gate, x digit planes) -> pf_group (positions per expert) -> pf_gateup
 // (gate/up + SwiGLU) -> pf_digits (h as digit planes) -> pf_down -> pf_combine.
 #include "moe_common.h"
+#include "split_mm.h"
 
 #include <stdio.h>
 #include <string.h>
@@ -381,33 +382,14 @@ __device__ __forceinline__ void pf_wgroups(uint4 (&d)[4]) {
     pf_swap(d[2], d[3]);   // groups 4 S + 2, 4 S + 3
 }
 
-// Dense GEMM over S rows of x (prefill projections, c/shaders/qmatmul_mm.comp): Y[s][o] =
-// sum_i x[s][i] W[o][i] for an fmt6 tensor of group size 128.  A unit is 128 output rows
-// (two 16-row tiles per wave) and one pass of <= 32 rows of x; the units of one row block
-// run on one XCD (workgroups go to the 8 XCDs round-robin), where their weights stay in L2.
-struct GemmArgs {
-    const uint8_t *w;       // lanes layout
-    const float *sz;        // [O][I / 128] [scale, zero]
-    int O, I, rb, nl;
-    const int8_t *xd;       // x digit planes [3][S][I]
-    const int *xe;          // [S][I / 128]
-    const float *xsum;
-    int S, nu, npass;       // rows of x; row blocks ceil(O / 128); passes ceil(S / 32)
-    float *y;               // [S][O]
-};
-constexpr int kGR = 2 * kGU;   // dense: output rows per unit
-
-// Gate/up + SwiGLU (kDense false) and the dense GEMM (kDense true) share one body.
-// MoE unit = 64 columns of h: wave w owns gate and up rows 64 u + 16 w .. + 15.  Dense unit
-// = 128 rows: wave w owns rows 128 u + 16 w + 64 m .. + 15 (m = 0, 1) in place of gate and up.
-// Per pass of <= 32 rows of x, supersteps of 4 groups: the x digit planes of the pass's rows
-// for the superstep sit in LDS (each thread stages its row's 12 x 16 bytes), the next
+// Gate/up + SwiGLU.  A unit is 64 columns of h: wave w owns gate and up rows 64 u + 16 w ..
+// + 15.  Per pass of <= 32 rows of x, supersteps of 4 groups: the x digit planes of the pass's
+// rows for the superstep sit in LDS (each thread stages its row's 12 x 16 bytes), the next
 // superstep's x digits and then its weight slots are loaded while this one computes, so the
 // in-order wait for those x digits never covers the weights.  Each (matrix, digit, 16-row
-// tile) is two MFMAs per group, folded in fp32 with the group's scale.  MoE: h = silu(gate) *
-// up (c/qwen.c:780-786, silu c/qwen.c:173) goes out as fp32 rows; dense: the two row tiles.
-template <bool kDense>
-__device__ __forceinline__ void gu_body(const PfArgs &a, const GemmArgs &g) {
+// tile) is two MFMAs per group, folded in fp32 with the group's scale; h = silu(gate) * up
+// (c/qwen.c:780-786, silu c/qwen.c:173) goes out as fp32 rows.
+__global__ __launch_bounds__(kPT, 2) void pf_gateup(PfArgs a) {
     __shared__ __attribute__((aligned(16))) int8_t sB[4][3][kPR][kPitch];
     __shared__ int sE[4][kPR];
     __shared__ float sQ[4][kPR];
@@ -420,29 +402,7 @@ __device__ __forceinline__ void gu_body(const PfArgs &a, const GemmArgs &g) {
     uint32_t abase, a1off, whalf;   // matrix 1's slots at abase + a1off
     const float2 *sgp, *sup;
     int nv[2];   // valid scale entries of the two matrices' unit rows
-    if constexpr (kDense) {
-        const int b = blockIdx.x, r = b >> 3;
-        u = 8 * (r / g.npass) + (b & 7);
-        if (u >= g.nu) return;
-        p0 = r % g.npass;
-        p1 = p0 + 1;
-        pos0 = 0;
-        n = g.S;
-        ngD = g.I / kGS;
-        xD = g.I;
-        xS = g.S;
-        const __amdgpu_buffer_rsrc_t w = buf_rsrc(g.w, (uint32_t)g.O * g.rb);
-        wr[0] = wr[1] = w;
-        const int row0 = u * kGR + wave * 16 + j;
-        abase = (uint32_t)(row0 * g.rb + q * 16);
-        a1off = (uint32_t)(kGU * g.rb);
-        whalf = (uint32_t)g.nl * 16;
-        sgp = (const float2 *)g.sz + (size_t)u * kGR * ngD;
-        sup = sgp + (size_t)kGU * ngD;
-        nv[0] = min(max(g.O - u * kGR, 0), kGU) * ngD;
-        nv[1] = min(max(g.O - u * kGR - kGU, 0), kGU) * ngD;
-        xr = buf_rsrc(g.xd, (uint32_t)(3u * g.S * g.I));
-    } else {
+    {
         ExpertRec rec;
         if (!pf_unit(a, a.I / kGU, e, u, p0, p1, pos0, n, rec)) return;
         ngD = a.D / kGS;
@@ -459,8 +419,8 @@ __device__ __forceinline__ void gu_body(const PfArgs &a, const GemmArgs &g) {
         xr = buf_rsrc(a.xd, (uint32_t)(3u * a.S * a.D));
     }
     const int nss = (ngD + 3) / 4;
-    const int *xe = kDense ? g.xe : a.xe;
-    const float *xsum = kDense ? g.xsum : a.xsum;
+    const int *xe = a.xe;
+    const float *xsum = a.xsum;
     // scales of the unit's rows of the two matrices, regrouped by group in LDS: the first kSV
     // entries per thread are loaded with the first pass's x row and weights
     constexpr int kSV = 2;
@@ -488,8 +448,7 @@ __device__ __forceinline__ void gu_body(const PfArgs &a, const GemmArgs &g) {
         // the scales (first pass), then the x digits once the row is known
         const int xi = r0 + min(sr, nr - 1);
         int xrow;
-        if constexpr (kDense) xrow = xi;
-        else xrow = a.units ? a.plist[pos0 + xi] : e == a.E ? xi : a.plist[pos0 + xi] / a.K;
+        xrow = a.units ? a.plist[pos0 + xi] : e == a.E ? xi : a.plist[pos0 + xi] / a.K;
         uint4 W[2][4];
         w_load(0, W);
         float2 sv[kSV][2];
@@ -607,20 +566,7 @@ __device__ __forceinline__ void gu_body(const PfArgs &a, const GemmArgs &g) {
             for (int tt = 0; tt < 2; tt++) {
                 const int x = tt * 16 + j;
                 if (tt >= NT || x >= nr) continue;
-                if constexpr (kDense) {
-                    // rows 128 u + 64 m + 16 w + 4 q .. + 3 of x row r0 + x
-#pragma unroll
-                    for (int m = 0; m < 2; m++) {
-                        const int row = u * kGR + m * kGU + wave * 16 + 4 * q;
-                        float *yr = g.y + (size_t)(r0 + x) * g.O + row;
-                        if (row + 3 < g.O && (g.O & 3) == 0)
-                            *(float4 *)yr = make_float4(facc[m][tt][0], facc[m][tt][1], facc[m][tt][2], facc[m][tt][3]);
-                        else
-#pragma unroll
-                            for (int r = 0; r < 4; r++)
-                                if (row + r < g.O) yr[r] = facc[m][tt][r];
-                    }
-                } else {
+                {
                     // h columns kGU u + 16 w + 4 q .. + 3 of x row tt * 16 + j
                     float hv[4];
 #pragma unroll
@@ -638,9 +584,6 @@ __device__ __forceinline__ void gu_body(const PfArgs &a, const GemmArgs &g) {
         __syncthreads();   // the next pass restages sB
     }
 }
-
-__global__ __launch_bounds__(kPT, 2) void pf_gateup(PfArgs a) { gu_body<false>(a, GemmArgs{}); }
-__global__ __launch_bounds__(kPT, 2) void gemm6_mfma(GemmArgs g) { gu_body<true>(PfArgs{}, g); }
 
 // Rows of n values (n % 128 == 0) -> digit planes [3][rows][n], ge / gsum [rows][n / 128]:
 // one thread per 8 columns.  kGated: the row is first put through the GatedDeltaNet output
@@ -833,6 +776,109 @@ __global__ __launch_bounds__(kPT, 2) void pf_down(PfArgs a) {
     }
 }
 
+// Rows of n values (n % 128 == 0) -> split planes (split_mm.h) [rows][n / 128][512 bytes] and
+// (p, sum) [rows][n / 128]: one thread per 8 columns.  kGated: the row is first put through
+// the GatedDeltaNet output norm, per head of VD columns y * r_h * gnorm[d] * silu(z) with
+// r_h = 1 / sqrt(mean(y^2) + eps), the sum of squares in double (c/qwen.c:768-772); gnorm
+// has a row stride (the host packs it into each token's parameter row).  VD / 8 consecutive
+// lanes hold one head (VD a power of two, 8 <= VD <= 512), so the head sum is a butterfly.
+template <bool kGated>
+__global__ __launch_bounds__(256) void pf_split_t(const float *__restrict__ src, int rows, int n,
+                                                  uint8_t *__restrict__ planes, float2 *__restrict__ xp,
+                                                  const float *__restrict__ z, const float *__restrict__ gnorm,
+                                                  int gstride, int VD, float eps) {
+    const int per = n / 8, i = blockIdx.x * 256 + threadIdx.x, row = i / per, c8 = i - row * per;
+    const bool valid = row < rows;
+    float v[8];
+    if (valid) {
+        const float4 a = *(const float4 *)(src + (size_t)row * n + 8 * c8),
+                     b = *(const float4 *)(src + (size_t)row * n + 8 * c8 + 4);
+        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+    } else {
+#pragma unroll
+        for (int c = 0; c < 8; c++) v[c] = 0.f;
+    }
+    if constexpr (kGated) {
+        double ss = 0;
+#pragma unroll
+        for (int c = 0; c < 8; c++) ss += (double)v[c] * v[c];
+        for (int o = 1; o < VD / 8; o <<= 1) ss += __shfl_xor(ss, o);
+        const float r = 1.f / sqrtf((float)(ss / VD) + eps);
+        if (valid) {
+            const float *zr = z + (size_t)row * n + 8 * c8;
+            const float *gw = gnorm + (size_t)row * gstride + (8 * c8) % VD;
+#pragma unroll
+            for (int c = 0; c < 8; c++) {   // silu(z) with a hardware reciprocal (< 2 ulp)
+                const float zv = zr[c], sz = zv * __builtin_amdgcn_rcpf(1.f + expf(-zv));
+                v[c] = v[c] * r * gw[c] * sz;
+            }
+        }
+    }
+    const size_t g = (size_t)(valid ? row : 0) * (n / kSmGS) + (8 * c8) / kSmGS;
+    sm_row8(v, valid, c8 & 15, planes + g * 512, xp + g);
+}
+
+// Dense GEMM over S rows of x (prefill projections, c/shaders/qmatmul_mm.comp): Y[s][o] =
+// sum_i x[s][i] W[o][i] for an fmt6 tensor of group size 128.  A block is RW * 32 output rows
+// by NT * 32 rows of x; the blocks of one row range run on one XCD (workgroups go to the 8
+// XCDs round-robin), where their weights stay in L2.
+struct GemmArgs {
+    const uint8_t *w;       // lanes layout
+    const float *sz;        // [O][I / 128] [scale, zero]
+    int O, I, rb, nl;
+    const uint8_t *xs;      // split planes of x [S][I / 128][512]
+    const float2 *xp;       // [S][I / 128]
+    int S, nu, npass;       // rows of x; row ranges; passes of NT * 32 rows of x
+    float *y;               // [S][O]
+};
+
+template <int RW, int KW, int NT>
+__global__ __launch_bounds__(RW * KW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm6_split(GemmArgs g) {
+    __shared__ SmLds<RW, KW, NT> L;
+    const int b = blockIdx.x, r = b >> 3, u = 8 * (r / g.npass) + (b & 7), pass = r % g.npass;
+    if (u >= g.nu) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rw = wave % RW, kw = wave / RW, row0 = u * RW * 32, x0 = pass * NT * 32, ng = g.I / kSmGS;
+    SmSrc<RW, KW, NT> src;
+    src.wr[0] = src.wr[1] = buf_rsrc(g.w, (uint32_t)g.O * g.rb);
+    src.xr = buf_rsrc(g.xs, (uint32_t)g.S * g.I * 4u);
+    src.half = (uint32_t)g.nl * 16u;
+    src.ng = ng;
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+        const int row = row0 + rw * 32 + m * 16 + (lane & 15);
+        src.wo[m] = row < g.O ? (uint32_t)row * g.rb : kOOB;
+    }
+#pragma unroll
+    for (int k = 0; k < SmSrc<RW, KW, NT>::kRows; k++) {
+        const int x = x0 + sm_stage_row<RW, KW, NT>(k);
+        src.xo[k] = x < g.S ? (uint32_t)x * g.I * 4u : kOOB;
+    }
+    const int srow = row0 + (threadIdx.x - kw * RW * 64) % (RW * 32);
+    src.scales(g.sz, min(srow, g.O - 1));
+#pragma unroll
+    for (int t = 0; t < NT; t++) src.xp[t] = g.xp + (size_t)min(x0 + t * 32 + (lane & 31), g.S - 1) * ng;
+    sm_f16 acc[NT];
+    sm_product<RW, KW, NT>(L, src, acc);
+    if (kw) return;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const int x = x0 + t * 32 + (lane & 31);
+        if (x >= g.S) continue;
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+            const int row = row0 + rw * 32 + 8 * r4 + 4 * (lane >> 5);
+            float *yr = g.y + (size_t)x * g.O + row;
+            if (row + 3 < g.O && (g.O & 3) == 0)
+                *(float4 *)yr = make_float4(acc[t][4 * r4], acc[t][4 * r4 + 1], acc[t][4 * r4 + 2], acc[t][4 * r4 + 3]);
+            else
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (row + i < g.O) yr[i] = acc[t][4 * r4 + i];
+        }
+    }
+}
+
 // ---------------------------------------------------------------- combine
 // out[t] = sum over t's K experts in ascending expert id of w * y[pos] + shgt * y_sh[t]
 // (c/qwen.c:1144, 1159-1161).  The token's ids, positions and weights come in one round of
@@ -985,7 +1031,36 @@ static PfScratch g_gm;
 
 bool gemm6_ok(const ColiVkTensor *t) {
     return tensor_live(t) && t->fmt == 6 && t->layout == kLayoutLanes && t->gs == kGS && t->I % kGS == 0 &&
-           t->I <= kGemmMaxI && t->O >= 1 && (size_t)(t->O + kGR) * t->row_bytes < (1ull << 32);
+           t->I <= kGemmMaxI && t->O >= 1 && (size_t)(t->O + 128) * t->row_bytes < (1ull << 32);
+}
+
+template <int RW, int KW, int NT>
+static bool gemm6_launch(GemmArgs &g, int min_blocks, hipStream_t st) {
+    g.nu = (g.O + RW * 32 - 1) / (RW * 32);
+    g.npass = (g.S + NT * 32 - 1) / (NT * 32);
+    if ((long)g.nu * g.npass < min_blocks) return false;
+    hipLaunchKernelGGL((gemm6_split<RW, KW, NT>), dim3(8 * ((g.nu + 7) / 8) * g.npass), dim3(RW * KW * 64), 0, st, g);
+    return true;
+}
+
+// The largest tile that still gives most CUs a block: 256 rows x 64 of x moves the fewest x
+// planes; fewer rows and 32 of x fill the chip sooner, with the groups split over the block's
+// waves where there are enough of them.  us per call, digits included (O x I x S; tiles 256 x 64,
+// 128 x 32 unsplit, 128 x 32 in 2 parts, 64 x 32 in 2, 64 x 32 in 4; the int8 kernel before):
+//   8192 x 2048 x 512: 49.9, 58.5, 68.2, 69.8, 93.5; 56.2   4096 x 2048 x 777: 45.2, 55.0, 67, 64, 86; 57.2
+//   2048 x 4096 x 512: 62.6, 36.9, 34.4, 38.9, 45.0; 43.5   12288 x 512 x 100: 16.1, 12.6, 15.0, 13.4, 22.2; 13.1
+//    512 x 2048 x 512: 38.5, 22.9, 21.1, 17.9, 18.2; 26.0    2048 x 4096 x 45: 56.4, 30.2, 25.7, 20.6, 19.1; 36.9
+//   8192 x 2048 x  45: 33.1, 18.7, 16.7, 14.4, 14.7; 21.8    2048 x 4096 x  8: 51.9, 28.5, 23.8, 19.1, 17.3; 25.4
+static void gemm6_dispatch(GemmArgs &g, hipStream_t st) {
+    const int cu = n_cu(), ng = g.I / kGS;
+    if (gemm6_launch<8, 1, 2>(g, cu * 5 / 8, st)) return;
+    if (ng <= 8) {
+        if (gemm6_launch<4, 1, 1>(g, cu * 3 / 4, st)) return;
+        gemm6_launch<2, 2, 1>(g, 0, st);
+    } else {
+        if (gemm6_launch<4, 2, 1>(g, cu * 3 / 4, st)) return;
+        gemm6_launch<2, 4, 1>(g, 0, st);
+    }
 }
 
 bool gemm6(const ColiVkTensor *const *t, float *const *d_y, int nt, const float *d_x, int S, hipStream_t st,
@@ -997,34 +1072,36 @@ bool gemm6(const ColiVkTensor *const *t, float *const *d_y, int nt, const float 
     if ((size_t)3 * S * I >= (1u << 31)) return false;
     if (gx && (!gx->z || !gx->gnorm || gx->VD < 8 || gx->VD > 512 || (gx->VD & (gx->VD - 1)) || I % gx->VD))
         return false;
-    const size_t o_xe = al256((size_t)3 * S * I), o_xs = o_xe + al256((size_t)S * ng * 4),
-                 total = o_xs + al256((size_t)S * ng * 4);
+    // rows per piece: the split planes (4 bytes a value) are addressed with 31-bit offsets
+    const int piece = min(S, (int)(((size_t)1 << 30) / ((size_t)4 * I)));
+    const size_t o_xp = al256((size_t)4 * piece * I), total = o_xp + al256((size_t)piece * ng * 8);
     if (!scratch(&g_gm.buf, &g_gm.cap, total)) return false;
     uint8_t *b = (uint8_t *)g_gm.buf;
-    const dim3 dg((unsigned)(((size_t)S * (I / 8) + 255) / 256));
-    if (gx)
-        hipLaunchKernelGGL(pf_digits_t<true>, dg, dim3(256), 0, st, d_x, S, I, (int8_t *)b, (int *)(b + o_xe),
-                           (float *)(b + o_xs), gx->z, gx->gnorm, gx->gstride, gx->VD, gx->eps);
-    else
-        hipLaunchKernelGGL(pf_digits_t<false>, dg, dim3(256), 0, st, d_x, S, I, (int8_t *)b, (int *)(b + o_xe),
-                           (float *)(b + o_xs), nullptr, nullptr, 0, 0, 0.f);
-    for (int i = 0; i < nt; i++) {
-        GemmArgs g;
-        g.w = t[i]->w;
-        g.sz = t[i]->sz;
-        g.O = t[i]->O;
-        g.I = I;
-        g.rb = t[i]->row_bytes;
-        g.nl = t[i]->nl;
-        g.xd = (const int8_t *)b;
-        g.xe = (const int *)(b + o_xe);
-        g.xsum = (const float *)(b + o_xs);
-        g.S = S;
-        g.nu = (g.O + kGR - 1) / kGR;
-        g.npass = (S + kPR - 1) / kPR;
-        g.y = d_y[i];
-        const int blocks = 8 * ((g.nu + 7) / 8) * g.npass;
-        hipLaunchKernelGGL(gemm6_mfma, dim3(blocks), dim3(kPT), (size_t)ng * 2 * kGU * sizeof(float2), st, g);
+    for (int s0 = 0; s0 < S; s0 += piece) {
+        const int n = min(piece, S - s0);
+        const dim3 dg((unsigned)(((size_t)n * (I / 8) + 255) / 256));
+        const float *x = d_x + (size_t)s0 * I;
+        if (gx)
+            hipLaunchKernelGGL(pf_split_t<true>, dg, dim3(256), 0, st, x, n, I, b, (float2 *)(b + o_xp),
+                               gx->z + (size_t)s0 * I, gx->gnorm + (size_t)s0 * gx->gstride, gx->gstride, gx->VD,
+                               gx->eps);
+        else
+            hipLaunchKernelGGL(pf_split_t<false>, dg, dim3(256), 0, st, x, n, I, b, (float2 *)(b + o_xp), nullptr,
+                               nullptr, 0, 0, 0.f);
+        for (int i = 0; i < nt; i++) {
+            GemmArgs g;
+            g.w = t[i]->w;
+            g.sz = t[i]->sz;
+            g.O = t[i]->O;
+            g.I = I;
+            g.rb = t[i]->row_bytes;
+            g.nl = t[i]->nl;
+            g.xs = b;
+            g.xp = (const float2 *)(b + o_xp);
+            g.S = n;
+            g.y = d_y[i] + (size_t)s0 * g.O;
+            gemm6_dispatch(g, st);
+        }
     }
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return fail("dense gemm launch", err);

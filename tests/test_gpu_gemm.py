@@ -72,6 +72,52 @@ def test_gemm_rows(lib, orc_omp, gen, O, I, S):
     _check(y, q, sz, x, S, I, O, gs, yo, f"gemm O={O} I={I} S={S}")
 
 
+@pytest.mark.parametrize("O,I,S", [(4, 128, 4), (100, 128, 31), (65, 384, 33), (2049, 1024, 97), (31, 1152, 64),
+                                   (6200, 1152, 130), (4100, 128, 641), (5121, 640, 515), (2560, 2176, 520)])
+def test_gemm_split_tiles(lib, gen, O, I, S):
+    """Every tile of the dense GEMM (256 x 64, 128 x 32, 64 x 32; whole, in 2 and in 4 parts of
+    the groups) at row counts just past and short of a tile, one group, odd group counts and
+    parts without a group, against the f64 product.  Per output the error is at most that of
+    the x planes (2^-23 of each x) and of the fp32 sums (16 steps in a group, then one per
+    group and part, each 2^-24 of the partial sum, and the scale's and zero's roundings), all
+    of them relative to sum |s| (|n - 8| + |z - 8|) |x|."""
+    gs = 128
+    q, sz = gen.fmt6(O, I, gs, 0x6E30 + O)
+    x = gen.normal(S * I, 0x6E31 + I)
+    y = lib.matmul(lib.tensor(q, sz, 6, I, O, gs), x, S=S).reshape(S, O)
+    y64 = _f64_rows(q, sz, x, S, I, O, gs)
+    b = q.reshape(O, I // 2)
+    nib = np.empty((O, I), np.float64)
+    nib[:, 0::2], nib[:, 1::2] = b & 15, b >> 4
+    s = sz.reshape(O, I // gs, 2).astype(np.float64)
+    w = (np.abs(nib.reshape(O, -1, gs) - 8) + np.abs(s[:, :, 1:2] - 8)) * np.abs(s[:, :, 0:1])
+    mag = np.abs(x.reshape(S, I).astype(np.float64)) @ w.reshape(O, I).T
+    bound = (2.0 ** -23 + (16 + I // gs + 8) * 2.0 ** -24) * mag
+    assert np.all(np.abs(y - y64) <= bound), float(np.max(np.abs(y - y64) / bound))
+
+
+def test_gemm_split_limits(lib, gen):
+    """Rows at the ends of the fp32 range: all zero, subnormal, near the largest number, and one
+    group 2^60 above the others; each row relative to its own product."""
+    O, I, gs = 96, 512, 128
+    q, sz = gen.fmt6(O, I, gs, 0x6E40)
+    x = gen.normal(8 * I, 0x6E41).reshape(8, I)
+    x[0] = 0.0
+    x[1] *= 2.0 ** -140
+    x[2] *= 2.0 ** -120
+    x[3] *= 2.0 ** 110
+    x[4, :gs] *= 2.0 ** 60
+    x[5, 1:] = 0.0
+    x = x.astype(np.float32)
+    y = lib.matmul(lib.tensor(q, sz, 6, I, O, gs), x.reshape(-1), S=8).reshape(8, O).astype(np.float64)
+    y64 = _f64_rows(q, sz, x.reshape(-1), 8, I, O, gs)
+    assert np.all(y[0] == 0.0)
+    for r in range(2, 8):
+        assert np.linalg.norm(y[r] - y64[r]) <= 2e-6 * np.linalg.norm(y64[r]), r
+    # 2^-140: x itself holds about 9 bits and the products round to multiples of 2^-149
+    assert np.max(np.abs(y[1] - y64[1])) <= 8 * 2.0 ** -149 * (I // gs)
+
+
 def test_gemm_wide_range_rows(lib, orc_omp, gen):
     """Rows of x whose groups span many binades (each group scaled by 2^k, k in -20..20):
     the per-(row, group) exponent of the digit decomposition follows each group."""
