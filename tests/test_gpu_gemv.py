@@ -56,6 +56,19 @@ def test_fmt6_shapes(lib, orc, gen, O, I, gs):
     assert normrel(y, yo) <= TOL_NORM
 
 
+@pytest.mark.parametrize("O,I,gs,S", [(8192, 2048, 128, 2), (4097, 512, 128, 3), (33, 2048, 64, 5), (9, 256, 32, 17),
+                                      (1, 128, 128, 2), (2500, 4096, 64, 33)])
+def test_fmt6_rows_one_launch(lib, gen, O, I, gs, S):
+    """Several rows of x on the GEMV (S < 4, or group sizes outside the dense GEMM) are one
+    launch for up to 16 rows: each row's bits are those of a call of its own."""
+    q, sz = gen.fmt6(O, I, gs, 2000 + O + I)
+    t = lib.tensor(q, sz, 6, I, O, gs)
+    x = gen.normal(S * I, gen.stream(I, O + S)).reshape(S, I)
+    y = lib.matmul(t, x.reshape(-1), S=S).reshape(S, O)
+    for s in range(S):
+        assert np.array_equal(y[s], lib.matmul(t, np.ascontiguousarray(x[s]))), s
+
+
 def test_fmt6_real_valued_zero(lib, orc, gen):
     """Startup RTN quantization gives non-integer zero points (c/qwen.c:246-265)."""
     O, I, gs = 256, 2048, 128
