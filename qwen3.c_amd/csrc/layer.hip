@@ -386,7 +386,10 @@ struct GdnArgs {
 
 // kTag (fused layer kernel): the inputs are polled from tagged words and y is published as
 // tagged words (the a/b path only; conv taps K <= kGdnMaxK).  bid: the block's index.
-template <int KPL, bool kTag>   // state elements per lane of a column (KD = 64 KPL)
+// AB: 0 decay / beta from params, the projection launch's dots or the general a/b loop; 1 / 2
+// the a/b rows (fmt 1 int8 / fmt 0 f32) over in_ln(resid) here, loaded with the state.
+constexpr int kAbWords = kLaneMaxI / 8 / kThreads;   // 8-column words per thread of the AB path
+template <int KPL, bool kTag, int AB>   // state elements per lane of a column (KD = 64 KPL)
 __device__ __forceinline__ void gdn_core_body(const GdnArgs &g, int bid) {
     __shared__ double s_red[kWaves];
     __shared__ float s_q[kGdnMaxKD], s_k[kGdnMaxKD], s_v[kGdnCols];
@@ -411,13 +414,42 @@ __device__ __forceinline__ void gdn_core_body(const GdnArgs &g, int bid) {
     const bool abp = !kTag && !g.params && g.ab;
     float pa, pb, pdtb, palog;
     {
-        const uint32_t nab = abp ? (uint32_t)g.VH * 8u : 0u, np = abp || kTag ? (uint32_t)g.VH * 4u : 0u;
+        const uint32_t nab = abp ? (uint32_t)g.VH * 8u : 0u, np = abp || kTag || AB ? (uint32_t)g.VH * 4u : 0u;
         const __amdgpu_buffer_rsrc_t ra = buf_rsrc(abp ? g.ab : g.dtb, nab), rd = buf_rsrc(g.dtb, np),
                                      rl = buf_rsrc(g.alog, np);
         pa = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra, h * 4, 0, 0));
         pb = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra, (g.VH + h) * 4, 0, 0));
         pdtb = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, h * 4, 0, 0));
         palog = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rl, h * 4, 0, 0));
+    }
+    // AB: the a/b rows of the head, the residual and the norm weight go out with them (read
+    // byte by byte after the conv and the norm they made it 14.8 us a launch, now 7); past D
+    // everything reads as zero
+    float axr[kAbWords][8], axw[kAbWords][8], asc = 1.f, bsc = 1.f;
+    uint4 aw[kAbWords][2], bw[kAbWords][2];
+    if constexpr (AB != 0) {
+        const __amdgpu_buffer_rsrc_t rx = buf_rsrc(g.resid, (uint32_t)g.D * 4u), rn = buf_rsrc(g.in_ln, (uint32_t)g.D * 4u);
+        const uint32_t eb = AB == 1 ? 1u : 4u;
+        const __amdgpu_buffer_rsrc_t rwa = buf_rsrc(g.a.w + (size_t)h * g.a.row_bytes, (uint32_t)g.D * eb),
+                                     rwb = buf_rsrc(g.b.w + (size_t)h * g.b.row_bytes, (uint32_t)g.D * eb);
+#pragma unroll
+        for (int k = 0; k < kAbWords; k++) {
+            const int w = tid + k * kThreads;
+            load8f(rx, w * 32, axr[k]);
+            load8f(rn, w * 32, axw[k]);
+            if constexpr (AB == 1) {
+                const float2 va = buf_load8f<kCached>(rwa, w * 8), vb = buf_load8f<kCached>(rwb, w * 8);
+                aw[k][0] = make_uint4(__float_as_uint(va.x), __float_as_uint(va.y), 0, 0);
+                bw[k][0] = make_uint4(__float_as_uint(vb.x), __float_as_uint(vb.y), 0, 0);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    aw[k][i] = buf_load16<kCached>(rwa, w * 32 + 16 * i);
+                    bw[k][i] = buf_load16<kCached>(rwb, w * 32 + 16 * i);
+                }
+            }
+        }
+        if (AB == 1) asc = g.a.sz[h], bsc = g.b.sz[h];
     }
 
     // conv1d + SiLU of the channels this block reads (c/qwen.c:697-707): q and k of the
@@ -510,10 +542,50 @@ __device__ __forceinline__ void gdn_core_body(const GdnArgs &g, int bid) {
         else s_v[t - 2 * KD] = v;
         if (t >= 2 * KD || owns_qk) g.ring[(size_t)g.head * g.CD + ch] = xn;
     }
+    if constexpr (AB != 0) {   // the norm's sum of squares
+        double ss = 0;
+#pragma unroll
+        for (int k = 0; k < kAbWords; k++)
+#pragma unroll
+            for (int c = 0; c < 8; c++) ss += (double)axr[k][c] * axr[k][c];
+        ss = wave_sum_dpp(ss);
+        if (lane == 0) s_red[wave] = ss;
+    }
     __syncthreads();
     // decay / beta (c/qwen.c:722-728): host params, the a/b dots of the projection launch, or
     // a/b over in_ln(resid) here (the fused kernel's came with the conv inputs)
     if (kTag) {
+    } else if constexpr (AB != 0) {   // the dots now, decay and beta after the next barrier
+        double ss = 0;
+        float da = 0.f, db = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) ss += s_red[w];
+        const float r = 1.f / sqrtf((float)(ss / g.D) + g.eps);
+#pragma unroll
+        for (int k = 0; k < kAbWords; k++)
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                float va, vb;
+                if constexpr (AB == 1) {
+                    const uint32_t ua = c < 4 ? aw[k][0].x : aw[k][0].y, ub = c < 4 ? bw[k][0].x : bw[k][0].y;
+                    va = (float)(int8_t)(ua >> (8 * (c & 3)));
+                    vb = (float)(int8_t)(ub >> (8 * (c & 3)));
+                } else {
+                    const uint4 ua = aw[k][c >> 2], ub = bw[k][c >> 2];
+                    const uint32_t a4[4] = {ua.x, ua.y, ua.z, ua.w}, b4[4] = {ub.x, ub.y, ub.z, ub.w};
+                    va = __uint_as_float(a4[c & 3]);
+                    vb = __uint_as_float(b4[c & 3]);
+                }
+                const float xv = axr[k][c] * r * (1.f + axw[k][c]);
+                da = fmaf(va, xv, da);
+                db = fmaf(vb, xv, db);
+            }
+        da = wave_sum_f(da);
+        db = wave_sum_f(db);
+        if (lane == 0) {
+            s_ab[0][wave] = da;
+            s_ab[1][wave] = db;
+        }
     } else if (g.params) {
         decay = g.params[h];
         beta = g.params[g.VH + h];
@@ -571,6 +643,18 @@ __device__ __forceinline__ void gdn_core_body(const GdnArgs &g, int bid) {
         }
     }
     __syncthreads();
+    if constexpr (AB != 0) {
+        float ta = 0.f, tb = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) {
+            ta += s_ab[0][w];
+            tb += s_ab[1][w];
+        }
+        const float sp_in = ta * asc + pdtb;
+        const float sp = sp_in > 20.f ? sp_in : log1pf(expf(sp_in));
+        decay = expf(-expf(palog) * sp);
+        beta = 1.f / (1.f + expf(-(tb * bsc)));
+    }
     const float rq = 1.f / sqrtf(s_nrm[0] + g.eps) / sqrtf((float)KD);
     const float rk = 1.f / sqrtf(s_nrm[1] + g.eps);
     float kq[KPL], qq[KPL];
@@ -612,9 +696,20 @@ __device__ __forceinline__ void gdn_core_body(const GdnArgs &g, int bid) {
     }
 }
 
-template <int KPL>
+template <int KPL, int AB>
 __global__ __launch_bounds__(kThreads) void gdn_core(GdnArgs g) {
-    gdn_core_body<KPL, false>(g, blockIdx.x);
+    gdn_core_body<KPL, false, AB>(g, blockIdx.x);
+}
+
+template <int AB>
+static bool gdn_core_launch(const GdnArgs &g, hipStream_t st) {
+    const dim3 grid(g.VH * (g.VD / kGdnCols));
+    switch (g.KD / 64) {
+    case 1: hipLaunchKernelGGL((gdn_core<1, AB>), grid, dim3(kThreads), 0, st, g); return true;
+    case 2: hipLaunchKernelGGL((gdn_core<2, AB>), grid, dim3(kThreads), 0, st, g); return true;
+    case 4: hipLaunchKernelGGL((gdn_core<4, AB>), grid, dim3(kThreads), 0, st, g); return true;
+    }
+    return false;
 }
 
 // ---------------------------------------------------------------- GDN over a chunk of tokens
@@ -2197,7 +2292,7 @@ __global__ __launch_bounds__(kThreads) void gdn_fused(GdnFusedArgs f) {
     __shared__ XPrep P;
     const int t = blockIdx.x;
     if (t < f.n1) proj_body<LPR1, kLaneChunks, kFuseU, XF_NORM, false, true>(f.p1, t, f.n1, P);
-    else if (t < f.n1 + f.nc) gdn_core_body<KPL, true>(f.g, t - f.n1);
+    else if (t < f.n1 + f.nc) gdn_core_body<KPL, true, 0>(f.g, t - f.n1);
     else proj_body<LPR3, kLaneChunks, kFuseU3, XF_GATED, true, false>(f.p3, t - f.n1 - f.nc, (int)gridDim.x - f.n1 - f.nc, P);
 }
 
@@ -2468,13 +2563,14 @@ static bool gdn_block(int gi, const float *src, const float *ln, const float *pa
     g.VD = d.VD;
     g.K = d.K;
     g.CD = d.CD;
-    const dim3 grid(d.VH * (d.VD / kGdnCols));
-    switch (d.KD / 64) {
-    case 1: hipLaunchKernelGGL(gdn_core<1>, grid, dim3(kThreads), 0, st, g); break;
-    case 2: hipLaunchKernelGGL(gdn_core<2>, grid, dim3(kThreads), 0, st, g); break;
-    case 4: hipLaunchKernelGGL(gdn_core<4>, grid, dim3(kThreads), 0, st, g); break;
-    default: return refuse("GDN key head dim not in {64, 128, 256}");
-    }
+    // int8 or f32 a/b rows (the engine's) over the normed residual: the vector path, for rows
+    // of whole 8-column words within its registers; other forms take the general loop
+    const int ab_rows = !params && !ab_proj && ln && ta->fmt == tb->fmt && (ta->fmt == 1 || ta->fmt == 0) && g.D % 8 == 0 &&
+                           g.D <= kLaneMaxI && ((uintptr_t)src & 15) == 0 && ((uintptr_t)ln & 15) == 0
+                       ? (ta->fmt == 1 ? 1 : 2)
+                       : 0;
+    if (!(ab_rows == 1 ? gdn_core_launch<1>(g, st) : ab_rows == 2 ? gdn_core_launch<2>(g, st) : gdn_core_launch<0>(g, st)))
+        return refuse("GDN key head dim not in {64, 128, 256}");
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail("GDN launch", e);
     G.head = G.head + 1 == G.K ? 0 : G.head + 1;   // the ring advanced by this token

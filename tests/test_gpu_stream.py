@@ -249,3 +249,22 @@ def test_stream_cfg3_geometry(lib, lorc, gen, moe_cfg):
         Vr = cache[1].reshape(W.KH, 4096, W.hd)[h, 4094:4096]
         assert np.max(np.abs(Kd - Kr)) <= 1e-4 * max(1.0, float(np.abs(Kr).max()))
         assert np.max(np.abs(Vd - Vr)) <= 1e-4 * max(1.0, float(np.abs(Vr).max()))
+
+
+@pytest.mark.parametrize("ab_fmt", [0, 1])
+def test_stream_rows_ab_cfg3(lib, lorc, gen, moe_cfg, ab_fmt):
+    """f32 and int8 a/b rows at configs[3] shapes (GatedDeltaNet layers only): the recurrence
+    launch takes their dots itself, whole rows of 2048 columns."""
+    L = moe_cfg
+    import _moe
+    _moe._active[0] = None
+    first = 66
+    lib.eg_table_init(first + 2, L.E, L.D, L.I, L.gs)
+    for l in range(first, first + 2):
+        L.register(lib, l)
+    gqa = dict(H=16, KH=2, hd=256, rot=64, gs=128)
+    gdn = dict(KH=16, KD=128, VH=32, VD=128, K=4, gs=128)
+    stack = _stack.Stack(lib, gen, 0xE620 + ab_fmt, 2, 2048, gqa, gdn, L, max_t=16, ab_fmt=ab_fmt, first_layer=first,
+                         state_base=115 + 2 * ab_fmt)
+    _run_stream(lib, lorc, stack, L.router, 8, 2, True, 0xE680 + ab_fmt, gen)
+    assert lib.moe_error() == 0
