@@ -30,6 +30,7 @@
 //               the sigmoid gate.
 #include "fmt6_device.h"
 #include "moe_common.h"
+#include "split_mm.h"
 
 #include <math.h>
 #include <stdio.h>
@@ -1796,8 +1797,8 @@ __global__ __launch_bounds__(kMT) void attn_merge_d(AttnArgs a) {
 // ---------------------------------------------------------------- GQA over S query rows
 // The block over S > 1 rows at positions pos_base .. pos_base + S - 1, causal (the prompt, or
 // a continuation chunk; c/qwen.c:581-667 restated, batched as c/backend_vulkan.c:2280-2340):
-// projections as GEMMs, qk_rows for the norms, RoPE and KV writes of all rows, attn_rows for
-// the attention and its output gate, then the o-projection GEMM.
+// projections as GEMMs, qk_rows for the norms, RoPE and KV writes of all rows, the attention
+// and its output gate, then the o-projection GEMM.
 
 // q/k norm + partial RoPE of one head row of token s (c/qwen.c:598-614, the arithmetic of
 // row_finish), block (s, j) of one wave: j < H is q head j into qn [S][H][hd]; j >= H is k
@@ -1851,144 +1852,301 @@ __global__ __launch_bounds__(64) void qk_rows(const float *__restrict__ qraw, co
     }
 }
 
-// Causal attention of 16 query rows of one head on fp32 MFMA (v_mfma_f32_16x16x4_f32), one
-// block of 4 waves per (head, 16-row query tile); wave w takes the key tiles w, w + 4, ...
-// of 16 positions and keeps its own running max, sum and context; the block merges the
-// four in wave order and applies the output gate (c/qwen.c:641-660).
-//   scores^T = K Q^T: A = 16 keys x 4 dims, B = 4 dims x 16 queries; lane l, register r of
-//     the product is (key 4 (l / 16) + r, query l % 16).  The K dimension is permuted: step
-//     kk of lane group g = l / 16 is dim (hd / 4) g + kk, so each lane holds a contiguous
-//     quarter of its query row (registers) and reads a contiguous quarter of its key row.
-//   ctx^T += V^T P^T: A = 16 dims x 4 keys (V tile from LDS), B = the lane's own 4 scores
-//     (step kk of group g is key 4 g + kk); lane l, register r of dim tile t is
-//     (dim 16 t + 4 (l / 16) + r, query l % 16).  Every per-query value (max, sum, rescale)
-//     stays in the lanes of its query.
-constexpr int kPQ = 16, kPKey = 16;
-struct AttnRowsArgs {
-    const float *qraw;    // [S][H][2 hd]: q | gate per head
-    const float *qn;      // [S][H][hd] normed, rotated
-    const float *Kc, *Vc; // [KH][max_t][hd]
-    float *ctx;           // [S][H hd] gated context
-    int S, H, KH, pos_base, max_t, nqt;
+// ---------------------------------------------------------------- attention over S rows, f16 MFMA
+// The same attention on v_mfma_f32_32x32x16_f16: every fp32 operand as two f16 planes (hi + lo,
+// 22 significant bits, scaled by powers of two), every product as hi hi + hi lo + lo hi summed
+// in fp32.  What is dropped, lo lo, is 2^-24 of the product, as an fp32 rounding.
+//   K, q: a power of two per row, taken out of the score.
+//   V, P: V' = V 2^-ev per key; the weight w = p 2^ev is scaled per query by the largest
+//     w so far (A, which decays with the softmax's rescaling as the context does), so what is
+//     lost of a weight is 2^-40 of the largest contribution to the query's context.
+// kv_split writes the planes of the call's keys once, in the order of the products' operands
+// (32 keys a tile): the query tiles of all heads then copy them to LDS as they are.
+//   scores^T = K q^T: A = 32 keys x 16 dims, B = 16 dims x 32 queries; lane l, register r is
+//     (key 8 (r / 4) + 4 (l / 32) + r % 4, query l % 32).
+//   ctx^T += V^T P^T: A = 32 dims x 16 keys, B = the lane's own 8 scores of registers 8 s ..
+//     8 s + 7, so V's operand holds key 16 s + 8 (j / 4) + 4 (l / 32) + j % 4 at element j.
+// One block is 4 waves that share the key tiles: 4 (2, 1) heads of one kv head by 1 (2, 4) tiles of
+// 32 query rows, over a part of the keys; attn_parts_merge joins the parts and applies the gate.
+// 96 products per 32 x 32 scores at hd 256; the fp32 products they replace took 5.3 times the
+// matrix cycles, and each wave read its own K rows from memory.
+// 1900 rows x 16 heads x 256 (2 kv heads): 209 us, the key planes 12 and the merge 41; the fp32
+// kernel 736.  Relative error of the layer against 64 bits 4.8e-7, before 1.1e-6.
+constexpr int kVm0 = 0x0F70;   // s_waitcnt vmcnt(0)
+constexpr int kSpT = 32;   // keys per tile, query rows per wave
+template <int HD>
+struct KvPlanes {
+    static constexpr int kUnits = HD / 16 * 2 * 64;   // 16-byte units of a tile's K; as many of V
+};
+
+template <int HD>
+__global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, const float *__restrict__ Vc, int max_t,
+                                                int nkeys, uint4 *__restrict__ planes, float *__restrict__ kscale,
+                                                int *__restrict__ vexp) {
+    __shared__ __attribute__((aligned(16))) float s_t[2][kSpT][HD + 4];
+    __shared__ int s_e[2][kSpT];
+    const int tile = blockIdx.x, kh = blockIdx.y, nt = gridDim.x, tid = threadIdx.x;
+    for (int i = tid; i < 2 * kSpT * (HD / 4); i += 256) {
+        const int m = i / (kSpT * (HD / 4)), key = i / (HD / 4) % kSpT, c4 = i % (HD / 4), t = tile * kSpT + key;
+        const float *src = (m ? Vc : Kc) + ((size_t)kh * max_t + t) * HD + 4 * c4;
+        *(float4 *)&s_t[m][key][4 * c4] = t < nkeys ? *(const float4 *)src : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    __syncthreads();
+    {   // 4 threads per row
+        const int m = tid >> 7, key = (tid >> 2) & 31, q = tid & 3;
+        float mx = 0.f;
+        for (int d = q; d < HD; d += 4) mx = fmaxf(mx, fabsf(s_t[m][key][d]));
+        mx = fmaxf(mx, __shfl_xor(mx, 1));
+        mx = fmaxf(mx, __shfl_xor(mx, 2));
+        if (q == 0) {
+            const int e = sm_exp(mx), o = (kh * nt + tile) * kSpT + key;
+            s_e[m][key] = e;
+            if (m) vexp[o] = mx == 0.f ? -300 : -e;   // a zero row has no weight
+            else kscale[o] = ldexpf(1.f, -e);
+        }
+    }
+    __syncthreads();
+    uint4 *dst = planes + (size_t)(kh * nt + tile) * 2 * KvPlanes<HD>::kUnits;
+    for (int i = tid; i < HD / 16 * 64; i += 256) {   // K: step i / 64, lane i % 64
+        const int st = i >> 6, l = i & 63, key = l & 31;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = ldexpf(s_t[0][key][16 * st + 8 * (l >> 5) + j], s_e[0][key]);
+        uint4 hi, lo;
+        sp_split8(v, hi, lo);
+        dst[(2 * st) * 64 + l] = hi;
+        dst[(2 * st + 1) * 64 + l] = lo;
+    }
+    for (int i = tid; i < HD / 32 * 2 * 64; i += 256) {   // V: dim tile, key step, lane
+        const int u = i >> 6, l = i & 63, d = (u >> 1) * 32 + (l & 31);
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int key = 16 * (u & 1) + 8 * (j >> 2) + 4 * (l >> 5) + (j & 3);
+            v[j] = ldexpf(s_t[1][key][d], s_e[1][key]);
+        }
+        uint4 hi, lo;
+        sp_split8(v, hi, lo);
+        dst[KvPlanes<HD>::kUnits + (2 * u) * 64 + l] = hi;
+        dst[KvPlanes<HD>::kUnits + (2 * u + 1) * 64 + l] = lo;
+    }
+}
+
+struct AttnSplitArgs {
+    const float *qn;       // [S][H][hd] normed, rotated
+    const uint4 *planes;   // [KH][ntile][K units | V units]
+    const float *kscale;   // [KH][ntile 32]
+    const int *vexp;
+    float *part;           // [S][H][np][hd] context sums of a part, relative to its maximum
+    float2 *ml;            // [S][H][np] (maximum, sum)
+    int S, H, KH, pos_base, ntile, hw, chunk, np;   // hw: heads per block; chunk: key tiles per part
     float scale;
 };
+
 template <int HD>
-__global__ __launch_bounds__(256) void attn_rows(AttnRowsArgs a) {
-    constexpr int NK = HD / 4, NDT = HD / 16, kVP = HD + 4;   // LDS pitch of a V row
-    __shared__ __attribute__((aligned(16))) float s_v[4][kPKey][kVP];
-    __shared__ float s_m[4][kPQ], s_l[4][kPQ];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = blockIdx.x % a.H, qt = a.nqt - 1 - blockIdx.x / a.H;   // the longest tiles first
-    const int G = a.H / a.KH, kh = h / G, qi = lane & 15, grp = lane >> 4;
-    const int s0 = qt * kPQ, sq = min(s0 + qi, a.S - 1), qpos = a.pos_base + sq;
-    const int last = a.pos_base + min(s0 + kPQ, a.S) - 1, nkt = last / kPKey + 1;
-    float qf[NK];
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void attn_split(AttnSplitArgs a) {
+    constexpr int NS = HD / 16, ND = HD / 32, kU = KvPlanes<HD>::kUnits, kLd = 2 * kU / 256;
+    constexpr int kRd = 3;   // operand reads run this many steps ahead of their products
+    __shared__ uint4 s_kv0[2 * kU], s_kv1[2 * kU];
+    __shared__ __attribute__((aligned(16))) float s_ks0[kSpT], s_ks1[kSpT];
+    __shared__ __attribute__((aligned(16))) int s_ve0[kSpT], s_ve1[kSpT];
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, col = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // block -> part, row block (the longest first), head group
+    const int G = a.H / a.KH, nhg = a.H / a.hw, rpb = 4 / a.hw, nrb = (a.S + kSpT * rpb - 1) / (kSpT * rpb);
+    const int hg = blockIdx.x % nhg, rb = nrb - 1 - blockIdx.x / nhg % nrb, p = blockIdx.x / nhg / nrb;
+    const int h = hg * a.hw + wave % a.hw, kh = hg * a.hw / G, s0 = (rb * rpb + wave / a.hw) * kSpT;
+    const int blast = (a.pos_base + min((rb + 1) * rpb * kSpT, a.S) - 1) / kSpT;   // last key tile of the block
+    const int t0 = p * a.chunk, t1 = min(t0 + a.chunk, blast + 1);
+    if (t0 >= t1) return;
+    const int wlast = s0 < a.S ? (a.pos_base + min(s0 + kSpT, a.S) - 1) / kSpT : -1;   // of the wave
+    const int sq = min(s0 + col, a.S - 1), qpos = a.pos_base + sq;
+    const uint4 *src = a.planes + (size_t)kh * a.ntile * 2 * kU;
+    // a tile straight to LDS (no registers: the q operands and the context take 256 of them); the
+    // two buffers are arrays of their own, so that the reads of one need not wait for the other's
+    // copies
+    auto copy = [&](int t, uint4 *dst, float *ks, int *ve) {
+        typedef const __attribute__((address_space(1))) void *gp;
+        typedef __attribute__((address_space(3))) void *lp;
+#pragma unroll
+        for (int i = 0; i < kLd; i++)
+            __builtin_amdgcn_global_load_lds((gp)(src + (size_t)t * 2 * kU + tid + 256 * i), (lp)(dst + 256 * i + wave * 64),
+                                             16, 0, 0);
+        if (tid < kSpT) {
+            __builtin_amdgcn_global_load_lds((gp)(a.kscale + (kh * a.ntile + t) * kSpT + tid), (lp)ks, 4, 0, 0);
+            __builtin_amdgcn_global_load_lds((gp)(a.vexp + (kh * a.ntile + t) * kSpT + tid), (lp)ve, 4, 0, 0);
+        }
+    };
+    // the wave's query rows as B operands
+    sm_h8 qh[NS], ql[NS];
+    float qs;
     {
-        const float4 *qp = (const float4 *)(a.qn + ((size_t)sq * a.H + h) * HD + NK * grp);
+        const float *qr = a.qn + ((size_t)sq * a.H + h) * HD + 8 * half;
+        float mx = 0.f;
 #pragma unroll
-        for (int i = 0; i < NK / 4; i++) {
-            const float4 v = qp[i];
-            qf[4 * i] = v.x, qf[4 * i + 1] = v.y, qf[4 * i + 2] = v.z, qf[4 * i + 3] = v.w;
-        }
-    }
-    coli_v4f acc[NDT];
+        for (int i = 0; i < NS; i++)
 #pragma unroll
-    for (int t = 0; t < NDT; t++) acc[t] = coli_v4f{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
-    const float *Kh = a.Kc + (size_t)kh * a.max_t * HD, *Vh = a.Vc + (size_t)kh * a.max_t * HD;
-    constexpr int kV4 = kPKey * HD / 4 / 64;   // float4 of the V tile per lane
-    for (int kt = wave; kt < nkt; kt += 4) {
-        const int t0 = kt * kPKey;
-        // key rows past the tile's last query position are masked; their loads stay inside
-        // the rows written so far (K clamped, V read as zeros: 0 * stale data is not 0)
-        float kf[NK];
-        const float4 *kp = (const float4 *)(Kh + (size_t)min(t0 + qi, last) * HD + NK * grp);
-#pragma unroll
-        for (int i = 0; i < NK / 4; i++) {
-            const float4 v = kp[i];
-            kf[4 * i] = v.x, kf[4 * i + 1] = v.y, kf[4 * i + 2] = v.z, kf[4 * i + 3] = v.w;
-        }
-        float4 vt[kV4];
-#pragma unroll
-        for (int i = 0; i < kV4; i++) {
-            const int f = lane + 64 * i, key = f / (HD / 4), c4 = f % (HD / 4);
-            vt[i] = t0 + key <= last ? *(const float4 *)(Vh + (size_t)(t0 + key) * HD + 4 * c4)
-                                     : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        coli_v4f sc = coli_v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < NK; kk++) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kk], qf[kk], sc, 0, 0, 0);
-        wave_lds_order();   // the previous tile's P.V reads of s_v come before these writes
-#pragma unroll
-        for (int i = 0; i < kV4; i++) {
-            const int f = lane + 64 * i, key = f / (HD / 4), c4 = f % (HD / 4);
-            *(float4 *)&s_v[wave][key][4 * c4] = vt[i];
-        }
-        // scale, causal mask, online softmax of the lane's query over the tile's 16 keys
-        float p[4], mx = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int kpos = t0 + 4 * grp + r;
-            p[r] = kpos <= qpos ? sc[r] * a.scale : -INFINITY;
-            mx = fmaxf(mx, p[r]);
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
+            for (int j = 0; j < 8; j++) mx = fmaxf(mx, fabsf(qr[16 * i + j]));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float mn = fmaxf(m, mx);
-        const bool live = mn != -INFINITY;   // some key of the query seen so far
-        const float al = live && m != -INFINITY ? expf(m - mn) : (live ? 0.f : 1.f);
-        float ps = 0.f;
+        const int e = sm_exp(mx);
+        qs = ldexpf(a.scale, -e);
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            p[r] = live && p[r] != -INFINITY ? expf(p[r] - mn) : 0.f;
-            ps += p[r];
+        for (int i = 0; i < NS; i++) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = ldexpf(qr[16 * i + j], e);
+            uint4 hi, lo;
+            sp_split8(v, hi, lo);
+            qh[i] = __builtin_bit_cast(sm_h8, hi);
+            ql[i] = __builtin_bit_cast(sm_h8, lo);
         }
-        ps += __shfl_xor(ps, 16);
-        ps += __shfl_xor(ps, 32);
-        l = l * al + ps;
-        m = mn;
-#pragma unroll
-        for (int t = 0; t < NDT; t++) acc[t] *= al;
-        wave_lds_order();   // the V tile is in LDS before the P.V reads (one wave: in order)
-#pragma unroll
-        for (int t = 0; t < NDT; t++)
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++)
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(s_v[wave][4 * grp + kk][16 * t + qi], p[kk], acc[t], 0,
-                                                              0, 0);
     }
-    // merge the four waves (wave order), gate, store
-    if (grp == 0) {
-        s_m[wave][qi] = m;
-        s_l[wave][qi] = l;
+    copy(t0, s_kv0, s_ks0, s_ve0);
+    __builtin_amdgcn_s_waitcnt(kVm0);
+    lds_barrier();
+    sm_f16 acc[ND];
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[d][r] = 0.f;
+    float m = -INFINITY, l = 0.f, A = 0.f;   // l: this lane's keys; A: the largest weight, R its exponent
+    int R = 0;
+    auto tile = [&](int t, const uint4 *K, const float *ks, const int *ve, uint4 *next, float *nks, int *nve) {
+        const int tn = min(t + 1, t1 - 1);   // the last tile is copied once more, into the free buffer
+        const uint4 *V = K + kU;
+        sm_f16 th;
+        copy(tn, next, nks, nve);   // their last reads are a barrier back
+        if (t <= wlast) {   // wave uniform
+#pragma unroll
+            for (int r = 0; r < 16; r++) th[r] = 0.f;
+            uint4 kf[kRd + 1][2];
+#pragma unroll
+            for (int i = 0; i < kRd; i++) kf[i][0] = K[(2 * i) * 64 + lane], kf[i][1] = K[(2 * i + 1) * 64 + lane];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < NS; i++) {
+                if (i + kRd < NS) {
+                    kf[(i + kRd) % (kRd + 1)][0] = K[(2 * (i + kRd)) * 64 + lane];
+                    kf[(i + kRd) % (kRd + 1)][1] = K[(2 * (i + kRd) + 1) * 64 + lane];
+                }
+                const sm_h8 kh8 = __builtin_bit_cast(sm_h8, kf[i % (kRd + 1)][0]),
+                            kl8 = __builtin_bit_cast(sm_h8, kf[i % (kRd + 1)][1]);
+                th = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl8, qh[i], th, 0, 0, 0);
+                th = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh8, ql[i], th, 0, 0, 0);
+                th = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh8, qh[i], th, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (t <= wlast) {
+            float pr[16], mx = -INFINITY;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; r4++) {
+                const float4 k4 = *(const float4 *)&ks[8 * r4 + 4 * half];
+                const float kk[4] = {k4.x, k4.y, k4.z, k4.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int r = 4 * r4 + i, kpos = t * kSpT + 8 * r4 + 4 * half + i;
+                    pr[r] = kpos <= qpos ? th[r] * (kk[i] * qs) : -INFINITY;
+                    mx = fmaxf(mx, pr[r]);
+                }
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const float mn = fmaxf(m, mx);
+            const bool live = mn != -INFINITY;   // some key of the query seen so far
+            const float al = live && m != -INFINITY ? expf(m - mn) : (live ? 0.f : 1.f);
+            float ps = 0.f, wm = 0.f;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; r4++) {
+                const int4 e4 = *(const int4 *)&ve[8 * r4 + 4 * half];
+                const int ee[4] = {e4.x, e4.y, e4.z, e4.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int r = 4 * r4 + i;
+                    const float e = live && pr[r] != -INFINITY ? expf(pr[r] - mn) : 0.f;
+                    ps += e;
+                    pr[r] = ldexpf(e, ee[i]);
+                    wm = fmaxf(wm, pr[r]);
+                }
+            }
+            l = l * al + ps;
+            m = mn;
+            wm = fmaxf(wm, __shfl_xor(wm, 32));
+            A = fmaxf(A * al, wm);
+            const int Rn = A > 0.f && A < INFINITY ? ilogbf(A) : R;
+            const float f = ldexpf(al, R - Rn);
+            R = Rn;
+            if (__ballot(f != 1.f) != 0ull)
+#pragma unroll
+                for (int d = 0; d < ND; d++) acc[d] *= f;
+            sm_h8 ph[2], pl[2];
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                float v[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = ldexpf(pr[8 * s + j], 14 - R);
+                uint4 hi, lo;
+                sp_split8(v, hi, lo);
+                ph[s] = __builtin_bit_cast(sm_h8, hi);
+                pl[s] = __builtin_bit_cast(sm_h8, lo);
+            }
+            uint4 vf[kRd + 1][2];   // step u: dim tile u / 2, keys 16 (u % 2) ..
+#pragma unroll
+            for (int u = 0; u < kRd; u++) vf[u][0] = V[(2 * u) * 64 + lane], vf[u][1] = V[(2 * u + 1) * 64 + lane];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 2 * ND; u++) {
+                if (u + kRd < 2 * ND) {
+                    vf[(u + kRd) % (kRd + 1)][0] = V[(2 * (u + kRd)) * 64 + lane];
+                    vf[(u + kRd) % (kRd + 1)][1] = V[(2 * (u + kRd) + 1) * 64 + lane];
+                }
+                const int d = u >> 1, s = u & 1;
+                const sm_h8 vh = __builtin_bit_cast(sm_h8, vf[u % (kRd + 1)][0]),
+                            vl = __builtin_bit_cast(sm_h8, vf[u % (kRd + 1)][1]);
+                acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph[s], acc[d], 0, 0, 0);
+                acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl[s], acc[d], 0, 0, 0);
+                acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[s], acc[d], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(kVm0);
+        lds_barrier();
+    };
+    for (int t = t0; t < t1; t += 2) {
+        tile(t, s_kv0, s_ks0, s_ve0, s_kv1, s_ks1, s_ve1);
+        if (t + 1 < t1) tile(t + 1, s_kv1, s_ks1, s_ve1, s_kv0, s_ks0, s_ve0);
     }
-    __syncthreads();
+    if (s0 + col >= a.S) return;
+    l += __shfl_xor(l, 32);
+    const size_t o = ((size_t)(s0 + col) * a.H + h) * a.np + p;
+    if (half == 0) a.ml[o] = make_float2(m, l);
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++)
+            *(float4 *)(a.part + o * HD + 32 * d + 8 * r4 + 4 * half) =
+                make_float4(ldexpf(acc[d][4 * r4], R - 14), ldexpf(acc[d][4 * r4 + 1], R - 14),
+                            ldexpf(acc[d][4 * r4 + 2], R - 14), ldexpf(acc[d][4 * r4 + 3], R - 14));
+}
+
+// Row s, head h: the parts' sums joined in key order, divided, gated (c/qwen.c:641-660).  Part p
+// exists when the row block's last key tile reaches it.
+template <int HD>
+__global__ __launch_bounds__(HD) void attn_parts_merge(AttnSplitArgs a, const float *__restrict__ qraw,
+                                                       float *__restrict__ ctx) {
+    const int s = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
+    const int last = (a.pos_base + s) / kSpT, n = last / a.chunk + 1;   // parts that hold keys of the row
+    const size_t o = ((size_t)s * a.H + h) * a.np;
     float M = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < 4; w++) M = fmaxf(M, s_m[w][qi]);
-    const float fw = m == -INFINITY ? 0.f : expf(m - M);
-    float (*s_c)[kPQ][HD] = (float (*)[kPQ][HD])&s_v[0][0][0];   // [4][16][HD] over the V tiles
-    static_assert(sizeof(s_v) >= 4 * kPQ * HD * 4, "context staging fits the V tiles");
-    __syncthreads();   // every wave is done with its V tile
-#pragma unroll
-    for (int t = 0; t < NDT; t++)
-        *(float4 *)&s_c[wave][qi][16 * t + 4 * grp] =
-            make_float4(acc[t][0] * fw, acc[t][1] * fw, acc[t][2] * fw, acc[t][3] * fw);
-    __syncthreads();
-    for (int o = tid; o < kPQ * HD; o += 256) {
-        const int q = o / HD, d = o % HD, s = s0 + q;
-        if (s >= a.S) continue;
-        float L = 0.f, Mq = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < 4; w++) Mq = fmaxf(Mq, s_m[w][q]);
-#pragma unroll
-        for (int w = 0; w < 4; w++) L += s_m[w][q] == -INFINITY ? 0.f : s_l[w][q] * expf(s_m[w][q] - Mq);
-        float c = 0.f;
-#pragma unroll
-        for (int w = 0; w < 4; w++) c += s_c[w][q][d];
-        const float gate = a.qraw[((size_t)s * a.H + h) * 2 * HD + HD + d];
-        a.ctx[(size_t)s * a.H * HD + (size_t)h * HD + d] = c / L * (1.f / (1.f + expf(-gate)));
+    for (int p = 0; p < n; p++) M = fmaxf(M, a.ml[o + p].x);
+    float L = 0.f, c = 0.f;
+    for (int p = 0; p < n; p++) {
+        const float2 v = a.ml[o + p];
+        const float f = v.x == -INFINITY ? 0.f : expf(v.x - M);
+        L += v.y * f;
+        if (f != 0.f) c += a.part[(o + p) * HD + d] * f;
     }
+    const float gate = qraw[((size_t)s * a.H + h) * 2 * HD + HD + d];
+    ctx[(size_t)s * a.H * HD + (size_t)h * HD + d] = c / L * (1.f / (1.f + expf(-gate)));
 }
 
 // ---------------------------------------------------------------- small kernels
@@ -2132,7 +2290,7 @@ static bool put_vec(float **d, int *have, const float *h, int n, const char *who
 // ---------------------------------------------------------------- work buffers
 enum {
     W_Q, W_K, W_V, W_CTX, W_PART, W_QKV, W_Z, W_Y, W_AB, W_NRM, W_LOGIT, W_IDX, W_IO_X, W_IO_R, W_IO_P, W_IO_O,
-    W_HIST, W_BND, W_SQKV, W_SZ, W_SY, W_ROPE, W_GQN, W_GKN, W_GVV, W_GMAT, W_COUNT
+    W_HIST, W_BND, W_SQKV, W_SZ, W_SY, W_ROPE, W_GQN, W_GKN, W_GVV, W_GMAT, W_APL, W_AKS, W_AVE, W_APT, W_AML, W_COUNT
 };
 struct WorkBuf {
     void *p = nullptr;
@@ -2768,8 +2926,8 @@ static int gqa_rows(int layer, const float *x, int D, ColiVkTensor *tq, ColiVkTe
     return read_back(out, dout, (size_t)S * Dout * 4, stream(), "gqa rows") ? 1 : 0;
 }
 
-// S >= kGemmMinS rows in one pass (c/backend_vulkan.c:2280-2340): q/k/v as one digit
-// decomposition and three GEMMs, qk_rows, attn_rows, the o-projection GEMM.  0 with no
+// S >= kGemmMinS rows in one pass (c/backend_vulkan.c:2280-2340): q/k/v as one split of x
+// and three GEMMs, qk_rows, the attention, the o-projection GEMM.  0 with no
 // device work done when a shape is outside these kernels (the caller then takes gqa_rows).
 enum { kSeqNo = -1 };
 static int g_gqa_seq = 1;   // 0: every S takes the token loop (coli_hip_gqa_seq)
@@ -2806,6 +2964,43 @@ static const float *rope_rows(float theta, int rot, int pos_end) {
     return c_tab.data();
 }
 
+// The attention of S rows: the key planes, the parts (about two blocks per CU, at least 4 key
+// tiles each), their merge.
+template <int HD>
+static bool attn_rows_split(const KvState &kv, const float *qn, const float *qraw, float *ctx, int S,
+                            const GqaDims &d, int pos_base, hipStream_t st) {
+    AttnSplitArgs a;
+    a.S = S;
+    a.H = d.H;
+    a.KH = d.KH;
+    a.pos_base = pos_base;
+    a.scale = 1.f / sqrtf((float)HD);
+    const int G = d.H / d.KH, nkeys = pos_base + S;
+    a.hw = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
+    a.ntile = (nkeys + kSpT - 1) / kSpT;
+    const int rows = kSpT * (4 / a.hw), nrb = (S + rows - 1) / rows, nhg = d.H / a.hw;
+    long steps = 0;
+    for (int r = 0; r < nrb; r++) steps += (pos_base + min((r + 1) * rows, S) - 1) / kSpT + 1;
+    const long want = (steps * nhg + 2 * n_cu() - 1) / (2 * n_cu());
+    a.chunk = max((int)want, max(4, (a.ntile + 15) / 16));
+    a.np = (a.ntile + a.chunk - 1) / a.chunk;
+    uint4 *planes = (uint4 *)wbuf(W_APL, (size_t)d.KH * a.ntile * 2 * KvPlanes<HD>::kUnits * 4);
+    float *ks = wbuf(W_AKS, (size_t)d.KH * a.ntile * kSpT);
+    int *ve = (int *)wbuf(W_AVE, (size_t)d.KH * a.ntile * kSpT);
+    a.part = wbuf(W_APT, (size_t)S * d.H * a.np * HD);
+    a.ml = (float2 *)wbuf(W_AML, (size_t)S * d.H * a.np * 2);
+    if (!planes || !ks || !ve || !a.part || !a.ml) return false;
+    a.qn = qn;
+    a.planes = planes;
+    a.kscale = ks;
+    a.vexp = ve;
+    hipLaunchKernelGGL(kv_split<HD>, dim3(a.ntile, d.KH), dim3(256), 0, st, kv.K, kv.V, d.max_t, nkeys, planes, ks, ve);
+    hipLaunchKernelGGL(attn_split<HD>, dim3((unsigned)((long)nhg * nrb * a.np)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(attn_parts_merge<HD>, dim3(S, d.H), dim3(HD), 0, st, a, qraw, ctx);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess || fail("attention rows launch", e);
+}
+
 static int gqa_seq(int layer, const float *x, int D, ColiVkTensor *tq, ColiVkTensor *tk, ColiVkTensor *tv,
                    ColiVkTensor *to, float *out, int S, const GqaDims &d, int pos_base, int Dout) {
     const int H = d.H, KH = d.KH, hd = d.hd, hr = d.rot / 2;
@@ -2835,25 +3030,10 @@ static int gqa_seq(int layer, const float *x, int D, ColiVkTensor *tq, ColiVkTen
     if (!gemm6(tp, yp, 3, dx, S, stream())) return 0;
     hipLaunchKernelGGL(qk_rows, dim3(S, H + KH), dim3(64), 0, stream(), qraw, kr, vr, qk.qn, qk.kn,
                        (const float2 *)rope, qn, kv.K, kv.V, H, KH, hd, d.rot, pos_base, d.max_t, d.eps);
-    AttnRowsArgs a;
-    a.qraw = qraw;
-    a.qn = qn;
-    a.Kc = kv.K;
-    a.Vc = kv.V;
-    a.ctx = ctx;
-    a.S = S;
-    a.H = H;
-    a.KH = KH;
-    a.pos_base = pos_base;
-    a.max_t = d.max_t;
-    a.nqt = (S + kPQ - 1) / kPQ;
-    a.scale = 1.f / sqrtf((float)hd);
-    const dim3 ga((unsigned)(H * a.nqt));
-    if (hd == 64) hipLaunchKernelGGL(attn_rows<64>, ga, dim3(256), 0, stream(), a);
-    else if (hd == 128) hipLaunchKernelGGL(attn_rows<128>, ga, dim3(256), 0, stream(), a);
-    else hipLaunchKernelGGL(attn_rows<256>, ga, dim3(256), 0, stream(), a);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail("attention rows launch", e) ? 1 : 0;
+    const bool ok2 = hd == 64 ? attn_rows_split<64>(kv, qn, qraw, ctx, S, d, pos_base, stream())
+                   : hd == 128 ? attn_rows_split<128>(kv, qn, qraw, ctx, S, d, pos_base, stream())
+                               : attn_rows_split<256>(kv, qn, qraw, ctx, S, d, pos_base, stream());
+    if (!ok2) return 0;
     const ColiVkTensor *op[1] = {to};
     float *const oy[1] = {dout};
     if (!gemm6(op, oy, 1, ctx, S, stream())) return 0;

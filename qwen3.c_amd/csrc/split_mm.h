@@ -71,6 +71,21 @@ __device__ __forceinline__ void sm_split8(const float (&v)[8], uint4 &hi, uint4 
     lo = b.u;
 }
 
+// 8 values (already scaled) -> their hi and lo units, in order
+__device__ __forceinline__ void sp_split8(const float (&v)[8], uint4 &hi, uint4 &lo) {
+    union {
+        _Float16 h[8];
+        uint4 u;
+    } a, b;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        a.h[k] = (_Float16)v[k];
+        b.h[k] = (_Float16)(v[k] - (float)a.h[k]);
+    }
+    hi = a.u;
+    lo = b.u;
+}
+
 // The power of two that brings a group with maximum m (>= 0) to [2^14, 2^15), as exponents:
 // x = v 2^-e, v = x 2^e.  Groups that are all zero or not finite keep 0; below 2^-135 the
 // exponent stops, so that 2^-e is still an fp32 number.

@@ -137,6 +137,46 @@ def test_gqa_full_rows(lib, lorc_omp, gen, shape):
         assert rel_to_max(Kd, Kr) < 1e-4 and rel_to_max(Vd, Vr) < 1e-5
 
 
+GQA_TILES = {   # D, H, KH, hd, rot, max_t, layer, S, pos_base: heads per block 1, 2 and 4; parts of the keys
+    "g1": (256, 4, 4, 64, 16, 400, 30, 65, 150),
+    "g3": (256, 6, 2, 64, 32, 400, 31, 33, 31),
+    "g2_hd128": (256, 4, 2, 128, 32, 400, 32, 97, 160),
+    "g4_hd256": (256, 4, 1, 256, 64, 700, 33, 31, 640),
+    "g8_hd256": (256, 8, 1, 256, 64, 64, 34, 64, 0),
+}
+
+
+@pytest.mark.parametrize("spread", [False, True])
+@pytest.mark.parametrize("shape", sorted(GQA_TILES))
+def test_gqa_row_tiles(lib, lorc_omp, gen, shape, spread):
+    """The attention over S rows at the edges of its 32-row and 32-key tiles, with the keys in
+    one and in several parts, every grouping of heads.  spread: cached rows whose values differ
+    by 2^40 (the largest on keys the queries hardly see) and one zero row, keys that differ by
+    2^8: each row is scaled on its own.  Against the oracle's token loop as test_gqa_full_rows."""
+    D, H, KH, hd, rot, max_t, layer, S, pos = GQA_TILES[shape]
+    layer += 10 * spread
+    W = _layers.GqaWeights(gen, gen.stream(0x9F40, layer), D, H, KH, hd, rot, 128)
+    tq, tk, tv, to = (m.upload(lib) for m in (W.q, W.k, W.v, W.o))
+    lib.kv_ensure(layer, KH * max_t, hd, hd)
+    lib.gqa_norm_weight(layer, W.qn, W.kn)
+    Kc = gen.normal(KH * max_t * hd, 0x9F50 + layer, 1.0).reshape(KH, max_t, hd)
+    Vc = gen.normal(KH * max_t * hd, 0x9F51 + layer, 1.0).reshape(KH, max_t, hd)
+    if spread:
+        Vc[:, 1::7] *= 2.0 ** -30
+        Vc[:, 2::9] = 0.0
+        Kc[:, 3::11] *= 2.0 ** -8
+        Vc[:, 5::50] *= 2.0 ** 10
+        Kc[:, 5::50] *= 2.0 ** -8
+    lib.kv_load(layer, 0, Kc.reshape(-1, hd), Vc.reshape(-1, hd))
+    cache = (Kc.reshape(-1).copy(), Vc.reshape(-1).copy())
+    xs = gen.normal(S * D, 0x9F60 + layer)
+    y = lib.gqa_full(layer, xs, tq, tk, tv, to, S, H, KH, hd, rot, pos, max_t, W.eps, W.theta)
+    for t in range(S):
+        ref = W.oracle(lorc_omp, cache, max_t, pos + t, xs[t * D:(t + 1) * D])
+        err = _util.maxrel_scaled(y[t * D:(t + 1) * D], ref)
+        assert err <= TOL, (t, err)
+
+
 # ---------------------------------------------------------------- GDN block
 host_params = _layers.gdn_host_params
 
