@@ -169,6 +169,125 @@ __global__ __launch_bounds__(256) void pf_logits(const float *__restrict__ xs, i
     if (t < S && e < E) lg[(size_t)t * E + e] = rfmt == 1 ? __fmul_rn(acc, rs[e]) : acc;
 }
 
+// The same sums for many rows, 4 tokens x 4 experts per 4x4 block: the sums on the VALU, the
+// products off the matrix cores.  v_mfma_f32_4x4x1 with C = 0 is 16 outer products of 4 values,
+// each x w + 0 rounded once, subnormals kept: it differs from a multiply only in the sign of a
+// zero, and a sum that starts at +0 never is -0, so adding either zero leaves it as it is.
+// pf_logits reads 32 bytes of LDS per 4 k of an output and is bound by that (2000 tokens x 256
+// experts x 2048: 117 us); here a wave owns 16 x 16 outputs, reads a quarter of it per output
+// and issues 5 instructions per k for 256 outputs instead of 8 (68 us).  A block of 2 x 2 waves
+// stages 32 rows of x and of w, KC columns at a time, double buffered, rows 4 banks apart;
+// columns past D are zeros on both sides and add +0.
+__global__ __launch_bounds__(256, 2) void pf_logits_mm(const float *__restrict__ xs, int S, int D,
+                                                       const uint8_t *__restrict__ rw, const float *__restrict__ rs,
+                                                       int rfmt, int rrb, int E, float *__restrict__ lg) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    constexpr int kR = 32, KC = 128, kC4 = KC / 4, kS = kR * kC4 / 256;   // kS: float4 staged per thread, x and w
+    constexpr int kRd = 3;
+    __shared__ __attribute__((aligned(16))) float s_x[2][kR][KC + 4];
+    __shared__ __attribute__((aligned(16))) float s_w[2][kR][KC + 4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wt = wave & 1, we = wave >> 1;
+    const int t0 = blockIdx.x * kR, e0 = blockIdx.y * kR;
+    float4 rx[kS], rv[kS];
+    auto load = [&](int kc) {
+#pragma unroll
+        for (int j = 0; j < kS; j++) {
+            const int i = tid + 256 * j, t = t0 + i / kC4, k = kc + 4 * (i % kC4);
+            rx[j] = (t < S && k < D) ? *(const float4 *)(xs + (size_t)t * D + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int j = 0; j < kS; j++) {
+            const int i = tid + 256 * j, e = e0 + i / kC4, k = kc + 4 * (i % kC4);
+            if (e >= E || k >= D) {
+                rv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+            } else if (rfmt == 0) {
+                rv[j] = *(const float4 *)(rw + (size_t)e * rrb + 4 * (size_t)k);
+            } else {
+                const char4 c = *(const char4 *)(rw + (size_t)e * rrb + k);
+                rv[j] = make_float4((float)c.x, (float)c.y, (float)c.z, (float)c.w);
+            }
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int j = 0; j < kS; j++) {
+            const int i = tid + 256 * j;
+            *(float4 *)&s_x[buf][i / kC4][4 * (i % kC4)] = rx[j];
+        }
+#pragma unroll
+        for (int j = 0; j < kS; j++) {
+            const int i = tid + 256 * j;
+            *(float4 *)&s_w[buf][i / kC4][4 * (i % kC4)] = rv[j];
+        }
+    };
+    // the lane's 4x4 block (4 by 4 of them), its operand rows, and after the products column
+    // lane & 3 of the block's 4 rows
+    const int xb = 16 * wt + 4 * (lane >> 4), xr = xb + (lane & 3);
+    const int wr = 16 * we + (lane & 15);
+    float acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc[j] = 0.f;
+    load(0);
+    store(0);
+    __syncthreads();
+    for (int kc = 0, buf = 0; kc < D; kc += KC, buf ^= 1) {
+        const bool more = kc + KC < D;
+        if (more) load(kc + KC);
+        // step n: four k; its operands are read kRd steps ahead, its products are made while the
+        // sums of step n - 1 run
+        float4 ra[kRd + 1], rw4[kRd + 1];
+        f4 p[2][4];
+        auto read = [&](int n) {
+            ra[n % (kRd + 1)] = *(const float4 *)&s_x[buf][xr][4 * n];
+            rw4[n % (kRd + 1)] = *(const float4 *)&s_w[buf][wr][4 * n];
+        };
+        auto mul = [&](int n, int c) {
+            const float a = ((const float *)&ra[n % (kRd + 1)])[c], w = ((const float *)&rw4[n % (kRd + 1)])[c];
+            const f4 z = {0.f, 0.f, 0.f, 0.f};
+            p[n & 1][c] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, w, z, 0, 0, 0);
+        };
+#pragma unroll
+        for (int n = 0; n < kRd; n++) read(n);
+#pragma unroll
+        for (int c = 0; c < 4; c++) mul(0, c);
+#pragma unroll
+        for (int n = 0; n < kC4; n++) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (n + kRd < kC4) read(n + kRd);
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                if (n + 1 < kC4) mul(n + 1, c);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    acc[j] = __fadd_rn(acc[j], p[n & 1][c][j]);
+                    if (c == 3) asm volatile("" : "+v"(acc[j]));   // the sums stay in their step
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (more) store(buf ^ 1);
+        __syncthreads();
+    }
+    const int e = e0 + wr;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int t = t0 + xb + j;
+        if (t < S && e < E) lg[(size_t)t * E + e] = rfmt == 1 ? __fmul_rn(acc[j], rs[e]) : acc[j];
+    }
+}
+
+// Below 3/4 of a wave of pf_logits_mm per SIMD its waves, alone on their SIMDs, issue too slowly:
+// 512 x 256 x 2048 30 us against 46, 768 rows about the same, 1024 rows 60 against 47.
+void logits_dispatch(const float *xs, int S, int D, const ColiVkTensor *t, float *lg, hipStream_t st) {
+    const int E = t->O;
+    if ((long)((S + 15) / 16) * ((E + 15) / 16) >= 3L * n_cu())
+        hipLaunchKernelGGL(pf_logits_mm, dim3((S + 31) / 32, (E + 31) / 32), dim3(256), 0, st, xs, S, D, t->w, t->sz,
+                           t->fmt, t->row_bytes, E, lg);
+    else
+        hipLaunchKernelGGL(pf_logits, dim3((S + kLT - 1) / kLT, (E + kLE - 1) / kLE), dim3(256), 0, st, xs, S, D, t->w,
+                           t->sz, t->fmt, t->row_bytes, E, lg);
+}
+
 // ---------------------------------------------------------------- route per token
 // One block per token: the routing (route_wave) of the token's reference logits, the
 // shared expert's gate sigmoid(x . sh_gate) (fp64 dot; c/qwen.c:1159), and x's digit
@@ -984,8 +1103,7 @@ bool moe_prefill(int layer, const ColiVkTensor *router, int K, const float *d_xs
     int *ti = d_idx ? d_idx : (int *)(b + o_ti), *off = (int *)(b + o_off);
     int *pl = (int *)(b + o_pl), *pp = (int *)(b + o_pp), *rk = (int *)(b + o_rk);
 
-    hipLaunchKernelGGL(pf_logits, dim3((S + kLT - 1) / kLT, (E + kLE - 1) / kLE), dim3(256), 0, st, d_xs, S, D,
-                       router->w, router->sz, router->fmt, router->row_bytes, E, lg);
+    logits_dispatch(d_xs, S, D, router, lg, st);
     PfArgs a;
     memset(&a, 0, sizeof(a));
     a.rec = rec;
@@ -1120,8 +1238,7 @@ bool gemm_f01_ok(const ColiVkTensor *t, const float *d_x) {
 
 bool gemm_f01(const ColiVkTensor *t, const float *d_x, float *d_y, int S, hipStream_t st) {
     if (!gemm_f01_ok(t, d_x) || S < 1 || !d_y) return false;
-    hipLaunchKernelGGL(pf_logits, dim3((S + kLT - 1) / kLT, (t->O + kLE - 1) / kLE), dim3(256), 0, st, d_x, S, t->I,
-                       t->w, t->sz, t->fmt, t->row_bytes, t->O, d_y);
+    logits_dispatch(d_x, S, t->I, t, d_y, st);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return fail("fmt 0/1 rows launch", err);
     return true;

@@ -165,6 +165,35 @@ def test_rows_f01(lib, orc, gen, fmt, O, I, S):
         assert np.array_equal(y[r], yo), (r, maxrel(y[r], yo))
 
 
+@pytest.mark.parametrize("fmt,O,I,S", [(0, 256, 132, 768), (0, 257, 260, 737), (1, 1000, 388, 197), (0, 33, 4, 4090)])
+def test_rows_f01_many(lib, orc, gen, fmt, O, I, S):
+    """Rows enough for the kernel with its products on the matrix cores: the same bits as the
+    sequential sums, also where the products are subnormal, zero of either sign or huge."""
+    x = gen.normal(S * I, 0x3110 + S).reshape(S, I)
+    x[1] *= np.float32(2.0 ** -126)
+    x[2] *= np.float32(2.0 ** -138)
+    x[3] = -0.0
+    x[4, ::3] = 0.0
+    x[5] *= np.float32(2.0 ** 110)
+    x[6, ::2] *= np.float32(2.0 ** -140)
+    x = np.ascontiguousarray(x.ravel())
+    if fmt == 1:
+        q, s = _int8_rows(orc, gen, O, I, 0x3111)
+        t = lib.tensor(q, s, 1, I, O, 0)
+    else:
+        W = gen.normal(O * I, 0x3112, 0.02)
+        t = lib.tensor(W, None, 0, I, O, 0)
+    y = lib.matmul(t, x, S).reshape(S, O)
+    for r in range(S):
+        yo = np.empty(O, np.float32)
+        xr = np.ascontiguousarray(x[r * I:(r + 1) * I])
+        if fmt == 1:
+            orc.orc_matmul_q8(P(yo), P(xr), P(q), P(s), I, O)
+        else:
+            orc.orc_matmul_f32(P(yo), P(xr), P(W), 1, I, O)
+        assert np.array_equal(y[r].view(np.uint32), yo.view(np.uint32)), (r, maxrel(y[r], yo))
+
+
 def test_rows_f01_pair(lib, orc, gen):
     """GatedDeltaNet b and a over S rows as one coli_vk_matmul_pair (c/qwen.c:1359), fmt 1."""
     S, I, VH = 37, 2048, 32
