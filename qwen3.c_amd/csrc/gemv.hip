@@ -836,7 +836,7 @@ COLI_API int coli_vk_matmul_pair(ColiVkTensor **t1p, float *y1, const void *w1, 
     float *dy = (float *)g_st.dy;
     const ColiVkTensor *tp[2] = {*t1p, *t2p};
     float *const yp[2] = {dy, dy + (size_t)S * O1};
-    if (S >= kGemmMinS && gemm6_ok(tp[0]) && gemm6_ok(tp[1])) {   // one digit decomposition of x for both
+    if (S >= kGemmMinS && gemm6_ok(tp[0]) && gemm6_ok(tp[1])) {   // one split of x for both
         if (!gemm6(tp, yp, 2, (const float *)g_st.dx, S, stream())) return 0;
     } else if (!gemv(tp[0], (const float *)g_st.dx, yp[0], S, stream()) ||
                !gemv(tp[1], (const float *)g_st.dx, yp[1], S, stream())) {

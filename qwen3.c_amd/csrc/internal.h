@@ -118,7 +118,7 @@ bool gemv_argmax(const ColiVkTensor *t, const float *d_x, float *d_y, hipStream_
 bool argmax_decode_host(const unsigned long long *keys, uint32_t epoch, int *idx, float *val);
 
 // Dense GEMM on MFMA over S rows of x (prefill.hip): d_y[i] [S][O_i] = x . t[i]^T for nt
-// fmt6 tensors of group size 128 sharing I (one digit decomposition of x serves all).  gx:
+// fmt6 tensors of group size 128 sharing I (one split of x serves all).  gx:
 // x is the GatedDeltaNet recurrence output and goes through its gated output norm first.
 constexpr int kGemmMaxI = kLaneMaxI;
 constexpr int kGemmMinS = 4;            // fewer rows of x: one GEMV launch per row

@@ -3152,7 +3152,7 @@ COLI_API int coli_vk_gdn_ba_weight(int layer, const float *alog, const float *dt
 
 // GDN prefill over S >= kGemmMinS tokens with host params (c/backend_vulkan.c:2018-2157),
 // per chunk of up to kGdnSeqChunk tokens: qkv and z of all the chunk's rows in one dense
-// GEMM (one digit decomposition of x), the recurrence of the chunk (gdn_chunk_prep /
+// GEMM (one split of x), the recurrence of the chunk (gdn_chunk_prep /
 // _mats / _scan over 64-token pieces; gdn_seq token by token for other shapes or when
 // coli_hip_gdn_chunked(0)), the ring push, then the gated norm and out-projection of all
 // rows in one more GEMM.

@@ -705,16 +705,10 @@ __global__ __launch_bounds__(kPT, 2) void pf_gateup(PfArgs a) {
 }
 
 // Rows of n values (n % 128 == 0) -> digit planes [3][rows][n], ge / gsum [rows][n / 128]:
-// one thread per 8 columns.  kGated: the row is first put through the GatedDeltaNet output
-// norm, per head of VD columns y * r_h * gnorm[d] * silu(z) with r_h = 1 / sqrt(mean(y^2)
-// + eps), the sum of squares in double (c/qwen.c:768-772); gnorm has a row stride (the
-// host packs it into each token's parameter row).  VD / 8 consecutive lanes hold one head
-// (VD a power of two, 8 <= VD <= 512), so the head sum is a butterfly over them.
-template <bool kGated>
-__global__ __launch_bounds__(256) void pf_digits_t(const float *__restrict__ src, int rows, int n,
-                                                   int8_t *__restrict__ planes, int *__restrict__ ge,
-                                                   float *__restrict__ gsum, const float *__restrict__ z,
-                                                   const float *__restrict__ gnorm, int gstride, int VD, float eps) {
+// one thread per 8 columns.
+__global__ __launch_bounds__(256) void pf_digits(const float *__restrict__ src, int rows, int n,
+                                                 int8_t *__restrict__ planes, int *__restrict__ ge,
+                                                 float *__restrict__ gsum) {
     const int per = n / 8, i = blockIdx.x * 256 + threadIdx.x, row = i / per, c8 = i - row * per;
     const bool valid = row < rows;
     float v[8];
@@ -725,22 +719,6 @@ __global__ __launch_bounds__(256) void pf_digits_t(const float *__restrict__ src
     } else {
 #pragma unroll
         for (int c = 0; c < 8; c++) v[c] = 0.f;
-    }
-    if constexpr (kGated) {
-        double ss = 0;
-#pragma unroll
-        for (int c = 0; c < 8; c++) ss += (double)v[c] * v[c];
-        for (int o = 1; o < VD / 8; o <<= 1) ss += __shfl_xor(ss, o);
-        const float r = 1.f / sqrtf((float)(ss / VD) + eps);
-        if (valid) {
-            const float *zr = z + (size_t)row * n + 8 * c8;
-            const float *gw = gnorm + (size_t)row * gstride + (8 * c8) % VD;
-#pragma unroll
-            for (int c = 0; c < 8; c++) {   // silu(z) with a hardware reciprocal (< 2 ulp)
-                const float zv = zr[c], sz = zv * __builtin_amdgcn_rcpf(1.f + expf(-zv));
-                v[c] = v[c] * r * gw[c] * sz;
-            }
-        }
     }
     const int ng = n / kGS, gi = (8 * c8) / kGS;
     const size_t r = valid ? row : 0;
@@ -1135,8 +1113,8 @@ bool moe_prefill(int layer, const ColiVkTensor *router, int K, const float *d_xs
     auto blocks = [&](int nu) { return ((nu * a.nsp + 7) & ~7) + nu * E8; };
     const int nh = I / kGU, nq = (D + kDR - 1) / kDR;
     hipLaunchKernelGGL(pf_gateup, dim3(blocks(nh)), dim3(kPT), (size_t)ngD * 2 * kGU * sizeof(float2), st, a);
-    hipLaunchKernelGGL(pf_digits_t<false>, dim3((P * (I / 8) + 255) / 256), dim3(256), 0, st, a.h, P, I,
-                       (int8_t *)(b + o_hd), (int *)(b + o_he), (float *)(b + o_hs), nullptr, nullptr, 0, 0, 0.f);
+    hipLaunchKernelGGL(pf_digits, dim3((P * (I / 8) + 255) / 256), dim3(256), 0, st, a.h, P, I,
+                       (int8_t *)(b + o_hd), (int *)(b + o_he), (float *)(b + o_hs));
     hipLaunchKernelGGL(pf_down, dim3(blocks(nq)), dim3(kPT), 0, st, a);
     hipLaunchKernelGGL(pf_combine, dim3(S), dim3(256), 0, st, a.y, ti, tv, tsh, pp, S, K, D, d_out);
     const hipError_t err = hipGetLastError();
@@ -1276,9 +1254,8 @@ bool eg_mfma(const PfUnit *d_units, int nunits, const int *d_xrow, int P, const 
     if (!scratch(&g_egx.buf, &g_egx.cap, ox_end)) return false;
     uint8_t *xb = (uint8_t *)g_egx.buf;
     if (key == 0 || key != g_egx_key || d_x != g_egx_src || Sx != g_egx_rows || D != g_egx_n || old != g_egx.buf) {
-        hipLaunchKernelGGL(pf_digits_t<false>, dim3((unsigned)(((size_t)Sx * (D / 8) + 255) / 256)), dim3(256), 0, st,
-                           d_x, Sx, D, (int8_t *)xb, (int *)(xb + ox_e), (float *)(xb + ox_s), nullptr, nullptr, 0, 0,
-                           0.f);
+        hipLaunchKernelGGL(pf_digits, dim3((unsigned)(((size_t)Sx * (D / 8) + 255) / 256)), dim3(256), 0, st,
+                           d_x, Sx, D, (int8_t *)xb, (int *)(xb + ox_e), (float *)(xb + ox_s));
         g_egx_key = key;
         g_egx_src = d_x;
         g_egx_rows = Sx;
@@ -1312,9 +1289,8 @@ bool eg_mfma(const PfUnit *d_units, int nunits, const int *d_xrow, int P, const 
     a.y = d_y;
     const int n8 = 8 * ((nunits + 7) / 8), nh = I / kGU, nq = (D + kDR - 1) / kDR;
     hipLaunchKernelGGL(pf_gateup, dim3(n8 * nh), dim3(kPT), (size_t)ngD * 2 * kGU * sizeof(float2), st, a);
-    hipLaunchKernelGGL(pf_digits_t<false>, dim3((unsigned)(((size_t)P * (I / 8) + 255) / 256)), dim3(256), 0, st, a.h,
-                       P, I, (int8_t *)(hb + oh_d), (int *)(hb + oh_e), (float *)(hb + oh_s), nullptr, nullptr, 0, 0,
-                       0.f);
+    hipLaunchKernelGGL(pf_digits, dim3((unsigned)(((size_t)P * (I / 8) + 255) / 256)), dim3(256), 0, st, a.h,
+                       P, I, (int8_t *)(hb + oh_d), (int *)(hb + oh_e), (float *)(hb + oh_s));
     hipLaunchKernelGGL(pf_down, dim3(n8 * nq), dim3(kPT), 0, st, a);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return fail("expert group mfma launch", err);
