@@ -1874,6 +1874,10 @@ __global__ __launch_bounds__(64) void qk_rows(const float *__restrict__ qraw, co
 // kernel 736.  Relative error of the layer against 64 bits 4.8e-7, before 1.1e-6.
 constexpr int kVm0 = 0x0F70;   // s_waitcnt vmcnt(0)
 constexpr int kSpT = 32;   // keys per tile, query rows per wave
+// Exponent of a V row with an infinity or NaN: its planes are zeros, and only the queries that
+// see the key give it a weight, an infinite one (so their context is NaN).  In the planes it
+// would reach the queries before it, whose weight 0 times it is NaN as well.
+constexpr int kVBad = 1 << 20;
 template <int HD>
 struct KvPlanes {
     static constexpr int kUnits = HD / 16 * 2 * 64;   // 16-byte units of a tile's K; as many of V
@@ -1895,13 +1899,20 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
     {   // 4 threads per row
         const int m = tid >> 7, key = (tid >> 2) & 31, q = tid & 3;
         float mx = 0.f;
-        for (int d = q; d < HD; d += 4) mx = fmaxf(mx, fabsf(s_t[m][key][d]));
+        int bad = 0;
+        for (int d = q; d < HD; d += 4) {
+            const float x = fabsf(s_t[m][key][d]);
+            mx = fmaxf(mx, x);
+            bad |= !(x < INFINITY);
+        }
         mx = fmaxf(mx, __shfl_xor(mx, 1));
         mx = fmaxf(mx, __shfl_xor(mx, 2));
+        bad |= __shfl_xor(bad, 1);
+        bad |= __shfl_xor(bad, 2);
         if (q == 0) {
             const int e = sm_exp(mx), o = (kh * nt + tile) * kSpT + key;
-            s_e[m][key] = e;
-            if (m) vexp[o] = mx == 0.f ? -300 : -e;   // a zero row has no weight
+            s_e[m][key] = m && bad ? kVBad : e;
+            if (m) vexp[o] = bad ? kVBad : mx == 0.f ? -300 : -e;   // a zero row has no weight
             else kscale[o] = ldexpf(1.f, -e);
         }
     }
@@ -1923,7 +1934,7 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const int key = 16 * (u & 1) + 8 * (j >> 2) + 4 * (l >> 5) + (j & 3);
-            v[j] = ldexpf(s_t[1][key][d], s_e[1][key]);
+            v[j] = s_e[1][key] == kVBad ? 0.f : ldexpf(s_t[1][key][d], s_e[1][key]);
         }
         uint4 hi, lo;
         sp_split8(v, hi, lo);
@@ -2064,7 +2075,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                     const int r = 4 * r4 + i;
                     const float e = live && pr[r] != -INFINITY ? expf(pr[r] - mn) : 0.f;
                     ps += e;
-                    pr[r] = ldexpf(e, ee[i]);
+                    pr[r] = ee[i] == kVBad ? (pr[r] == -INFINITY ? 0.f : INFINITY) : ldexpf(e, ee[i]);
                     wm = fmaxf(wm, pr[r]);
                 }
             }

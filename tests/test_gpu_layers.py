@@ -106,7 +106,7 @@ GQA_ROWS = {   # D, H, KH, hd, rot, gs, max_t, layer, S, pos_base, S2 (a continu
 @pytest.mark.parametrize("shape", sorted(GQA_ROWS))
 def test_gqa_full_rows(lib, lorc_omp, gen, shape):
     """coli_vk_gqa_full with S >= 4 rows: one batched pass (q/k/v and o-projection GEMMs on
-    MFMA, the norms, RoPE and KV writes of all rows, causal attention on fp32 MFMA) against
+    MFMA, the norms, RoPE and KV writes of all rows, causal attention on f16 MFMA) against
     the oracle's token loop (c/qwen.c:581-667), then a continuation call of S2 rows; cache
     rows before pos_base are seeded, partial 16-row query tiles occur; the KV rows the passes
     write against the oracle's cache."""
@@ -175,6 +175,27 @@ def test_gqa_row_tiles(lib, lorc_omp, gen, shape, spread):
         ref = W.oracle(lorc_omp, cache, max_t, pos + t, xs[t * D:(t + 1) * D])
         err = _util.maxrel_scaled(y[t * D:(t + 1) * D], ref)
         assert err <= TOL, (t, err)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("row", [0, 17, 31, 32, 64])
+def test_gqa_rows_nonfinite(lib, gen, row, bad):
+    """One row of x with a NaN or an infinity: the rows before it see none of it, also those
+    of its 32-row and 32-key tile (the same bits as with a finite row there), the rows from it
+    on are not finite (its key and value are in their sums, c/qwen.c:641-660)."""
+    D, H, KH, hd, rot, max_t, layer, S, pos = 256, 4, 2, 64, 16, 100, 50, 65, 0
+    W = _layers.GqaWeights(gen, gen.stream(0x9F70, layer), D, H, KH, hd, rot, 128)
+    tq, tk, tv, to = (m.upload(lib) for m in (W.q, W.k, W.v, W.o))
+    lib.kv_ensure(layer, KH * max_t, hd, hd)
+    lib.gqa_norm_weight(layer, W.qn, W.kn)
+    xs = gen.normal(S * D, 0x9F80 + row).copy()
+    y = [None, None]
+    for i in range(2):
+        if i:
+            xs[row * D + 5] = bad
+        y[i] = lib.gqa_full(layer, xs, tq, tk, tv, to, S, H, KH, hd, rot, pos, max_t, W.eps, W.theta).reshape(S, D).copy()
+    assert np.array_equal(y[0][:row], y[1][:row])
+    assert not np.isfinite(y[1][row:]).any(axis=1).any()
 
 
 # ---------------------------------------------------------------- GDN block
