@@ -277,10 +277,12 @@ __global__ __launch_bounds__(256, 2) void pf_logits_mm(const float *__restrict__
 }
 
 // Below 3/4 of a wave of pf_logits_mm per SIMD its waves, alone on their SIMDs, issue too slowly:
-// 512 x 256 x 2048 30 us against 46, 768 rows about the same, 1024 rows 60 against 47.
+// 512 x 256 x 2048 30 us against 46, 768 rows about the same, 1024 rows 60 against 47.  int8 rows,
+// converted as they are staged, from a whole wave: MoE block of 800 rows x 256 experts x 1024 190.8 us
+// against 192.0 here, 1030 rows 173.1 against 161.1 (I 512, 256), 1030 x 2048 296 against 271.
 void logits_dispatch(const float *xs, int S, int D, const ColiVkTensor *t, float *lg, hipStream_t st) {
     const int E = t->O;
-    if ((long)((S + 15) / 16) * ((E + 15) / 16) >= 3L * n_cu())
+    if ((long)((S + 15) / 16) * ((E + 15) / 16) >= (t->fmt == 1 ? 4L : 3L) * n_cu())
         hipLaunchKernelGGL(pf_logits_mm, dim3((S + 31) / 32, (E + 31) / 32), dim3(256), 0, st, xs, S, D, t->w, t->sz,
                            t->fmt, t->row_bytes, E, lg);
     else

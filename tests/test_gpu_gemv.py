@@ -165,7 +165,8 @@ def test_rows_f01(lib, orc, gen, fmt, O, I, S):
         assert np.array_equal(y[r], yo), (r, maxrel(y[r], yo))
 
 
-@pytest.mark.parametrize("fmt,O,I,S", [(0, 256, 132, 768), (0, 257, 260, 737), (1, 1000, 388, 197), (0, 33, 4, 4090)])
+@pytest.mark.parametrize("fmt,O,I,S", [(0, 256, 132, 768), (0, 257, 260, 737), (1, 1000, 388, 197), (0, 33, 4, 4090),
+                                         (1, 1000, 388, 262), (1, 257, 36, 993)])
 def test_rows_f01_many(lib, orc, gen, fmt, O, I, S):
     """Rows enough for the kernel with its products on the matrix cores: the same bits as the
     sequential sums, also where the products are subnormal, zero of either sign or huge."""
