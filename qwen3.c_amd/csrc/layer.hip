@@ -2154,7 +2154,7 @@ __global__ __launch_bounds__(HD) void attn_parts_merge(AttnSplitArgs a, const fl
         const float2 v = a.ml[o + p];
         const float f = v.x == -INFINITY ? 0.f : expf(v.x - M);
         L += v.y * f;
-        if (f != 0.f) c += a.part[(o + p) * HD + d] * f;
+        c += a.part[(o + p) * HD + d] * f;   // f = 0 too: a part that is not finite stays so
     }
     const float gate = qraw[((size_t)s * a.H + h) * 2 * HD + HD + d];
     ctx[(size_t)s * a.H * HD + (size_t)h * HD + d] = c / L * (1.f / (1.f + expf(-gate)));

@@ -198,6 +198,55 @@ def test_gqa_rows_nonfinite(lib, gen, row, bad):
     assert not np.isfinite(y[1][row:]).any(axis=1).any()
 
 
+# Rows of one block whose cached keys span several parts: 333 keys in parts of 128
+PARTS = dict(D=256, H=4, KH=2, hd=64, rot=16, max_t=400, S=33, pos=300)
+
+
+def _parts_block(lib, gen, layer, seed, weights=None):
+    """A block of PARTS with seeded weights (weights(W) may change them), its cache rows
+    [KH][max_t][hd] and a function that loads them and runs the rows."""
+    c = PARTS
+    W = _layers.GqaWeights(gen, gen.stream(0x9FA0, seed), c["D"], c["H"], c["KH"], c["hd"], c["rot"], 128)
+    if weights:
+        weights(W)
+    t = [m.upload(lib) for m in (W.q, W.k, W.v, W.o)]
+    shape = (c["KH"], c["max_t"], c["hd"])
+    Kc = gen.normal(int(np.prod(shape)), 0x9FB0 + seed).reshape(shape).copy()
+    Vc = gen.normal(int(np.prod(shape)), 0x9FB1 + seed).reshape(shape).copy()
+    xs = gen.normal(c["S"] * c["D"], 0x9FC0 + seed)
+
+    def run():
+        lib.kv_ensure(layer, c["KH"] * c["max_t"], c["hd"], c["hd"])
+        lib.gqa_norm_weight(layer, W.qn, W.kn)
+        lib.kv_load(layer, 0, Kc.reshape(-1, c["hd"]), Vc.reshape(-1, c["hd"]))
+        return lib.gqa_full(layer, xs, *t, c["S"], c["H"], c["KH"], c["hd"], c["rot"], c["pos"], c["max_t"], W.eps,
+                            W.theta).reshape(c["S"], c["D"]).copy()
+
+    def oracle(orc):
+        cache = (Kc.reshape(-1).copy(), Vc.reshape(-1).copy())
+        with np.errstate(all="ignore"):
+            return np.stack([W.oracle(orc, cache, c["max_t"], c["pos"] + s,
+                                      np.ascontiguousarray(xs[s * c["D"]:(s + 1) * c["D"]])) for s in range(c["S"])])
+    return Kc, Vc, run, oracle
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("far", [False, True])
+@pytest.mark.parametrize("row", [3, 64, 200, 299])
+def test_gqa_rows_cached_v_nonfinite(lib, gen, row, far, bad):
+    """One cached V row with a NaN or an infinity, every K finite: every query that sees the
+    key is not finite (its weight, 0 included, times such a value: c/qwen.c:654-658), whichever
+    part of the keys it lies in, also where the scores of its part are hundreds below the
+    row's maximum (far) and its weight underflows."""
+    Kc, Vc, run, _ = _parts_block(lib, gen, 150, 1)
+    Vc[1, row, 7] = bad
+    if far:
+        part = np.arange(Kc.shape[1]) // 128 == row // 128
+        Kc[:, ~part] *= 200.0
+    y = run()
+    assert not np.isfinite(y).any()
+
+
 # ---------------------------------------------------------------- GDN block
 host_params = _layers.gdn_host_params
 
