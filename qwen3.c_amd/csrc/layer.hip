@@ -2073,7 +2073,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const int r = 4 * r4 + i;
-                    const float e = live && pr[r] != -INFINITY ? expf(pr[r] - mn) : 0.f;
+                    const float e = pr[r] != -INFINITY ? expf(pr[r] - mn) : 0.f;   // NaN stays, also with no live key yet
                     ps += e;
                     pr[r] = ee[i] == kVBad ? (pr[r] == -INFINITY ? 0.f : INFINITY) : ldexpf(e, ee[i]);
                     wm = fmaxf(wm, pr[r]);

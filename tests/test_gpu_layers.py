@@ -247,6 +247,14 @@ def test_gqa_rows_cached_v_nonfinite(lib, gen, row, far, bad):
     assert not np.isfinite(y).any()
 
 
+@pytest.mark.parametrize("r0,r1", [(3, 4), (0, 32), (0, 128), (128, 300)])
+def test_gqa_rows_cached_k_nan(lib, gen, r0, r1):
+    """NaN K rows, whole tiles and parts of them: no query that sees one is finite."""
+    Kc, Vc, run, _ = _parts_block(lib, gen, 150, 5)
+    Kc[:, r0:r1, 9] = np.nan
+    assert not np.isfinite(run()).any()
+
+
 # ---------------------------------------------------------------- GDN block
 host_params = _layers.gdn_host_params
 
