@@ -32,6 +32,7 @@
 #include "moe_common.h"
 #include "split_mm.h"
 
+#include <float.h>
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -2084,7 +2085,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             wm = fmaxf(wm, __shfl_xor(wm, 32));
             A = fmaxf(A * al, wm);
             const int Rn = A > 0.f && A < INFINITY ? ilogbf(A) : R;
-            const float f = ldexpf(al, R - Rn);
+            const float f = fminf(ldexpf(al, R - Rn), FLT_MAX);   // past 2^128 only while the context is 0: stays 0
             R = Rn;
             if (__ballot(f != 1.f) != 0ull)
 #pragma unroll

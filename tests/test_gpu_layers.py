@@ -255,6 +255,25 @@ def test_gqa_rows_cached_k_nan(lib, gen, r0, r1):
     assert not np.isfinite(run()).any()
 
 
+def _no_v(W):
+    W.v.sz.reshape(-1, 2)[:, 0] = 0.0
+
+
+@pytest.mark.parametrize("zeros,exp", [(64, -110), (64, -120), (0, -100), (300, 0), (0, 100)])
+def test_gqa_rows_v_scales(lib, lorc_omp, gen, zeros, exp):
+    """Cached V rows near the ends of the fp32 range (the call's own rows are zero), after a run
+    of zero rows.  1e-4 of the output row's norm: on either side a 64-term score errs by up to
+    64 2^-24 sum |q k| / 8 (2e-5 at these values) and with it a weight, and the 256-term sums of
+    the output projection by 256 2^-24 of their terms (2e-5)."""
+    Kc, Vc, run, oracle = _parts_block(lib, gen, 150, 6, _no_v)
+    Vc[:, :zeros] = 0.0
+    Vc *= np.float32(2.0 ** exp)
+    y, ref = run().astype(np.float64), oracle(lorc_omp).astype(np.float64)
+    assert np.isfinite(y).all()
+    for s in range(len(y)):
+        assert np.linalg.norm(y[s] - ref[s]) <= 1e-4 * np.linalg.norm(ref[s]), s
+
+
 # ---------------------------------------------------------------- GDN block
 host_params = _layers.gdn_host_params
 
