@@ -1858,9 +1858,10 @@ __global__ __launch_bounds__(64) void qk_rows(const float *__restrict__ qraw, co
 // 22 significant bits, scaled by powers of two), every product as hi hi + hi lo + lo hi summed
 // in fp32.  What is dropped, lo lo, is 2^-24 of the product, as an fp32 rounding.
 //   K, q: a power of two per row, taken out of the score.
-//   V, P: V' = V 2^-ev per key; the weight w = p 2^ev is scaled per query by the largest
-//     w so far (A, which decays with the softmax's rescaling as the context does), so what is
-//     lost of a weight is 2^-40 of the largest contribution to the query's context.
+//   V, P: V' = V 2^(14-ev) per key, its largest element in [2^14, 2^15); the weight w = p 2^ev
+//     is about the key's contribution (no smaller than it in fp32, so tiny V keep their bits),
+//     scaled per query by the largest w so far (A, which decays with the softmax's rescaling as
+//     the context does): what is lost of a weight is at most 2^-39 of the largest.
 // kv_split writes the planes of the call's keys once, in the order of the products' operands
 // (32 keys a tile): the query tiles of all heads then copy them to LDS as they are.
 //   scores^T = K q^T: A = 32 keys x 16 dims, B = 16 dims x 32 queries; lane l, register r is
@@ -1913,7 +1914,7 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
         if (q == 0) {
             const int e = sm_exp(mx), o = (kh * nt + tile) * kSpT + key;
             s_e[m][key] = m && bad ? kVBad : e;
-            if (m) vexp[o] = bad ? kVBad : mx == 0.f ? -300 : -e;   // a zero row has no weight
+            if (m) vexp[o] = bad ? kVBad : mx == 0.f ? -300 : 14 - e;   // a zero row has no weight
             else kscale[o] = ldexpf(1.f, -e);
         }
     }
@@ -2136,8 +2137,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
         for (int r4 = 0; r4 < 4; r4++)
             *(float4 *)(a.part + o * HD + 32 * d + 8 * r4 + 4 * half) =
-                make_float4(ldexpf(acc[d][4 * r4], R - 14), ldexpf(acc[d][4 * r4 + 1], R - 14),
-                            ldexpf(acc[d][4 * r4 + 2], R - 14), ldexpf(acc[d][4 * r4 + 3], R - 14));
+                make_float4(ldexpf(acc[d][4 * r4], R - 28), ldexpf(acc[d][4 * r4 + 1], R - 28),
+                            ldexpf(acc[d][4 * r4 + 2], R - 28), ldexpf(acc[d][4 * r4 + 3], R - 28));
 }
 
 // Row s, head h: the parts' sums joined in key order, divided, gated (c/qwen.c:641-660).  Part p
