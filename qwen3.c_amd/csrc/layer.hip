@@ -1887,7 +1887,7 @@ struct KvPlanes {
 
 template <int HD>
 __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, const float *__restrict__ Vc, int max_t,
-                                                int nkeys, uint4 *__restrict__ planes, float *__restrict__ kscale,
+                                                int nkeys, uint4 *__restrict__ planes, int *__restrict__ kexp,
                                                 int *__restrict__ vexp) {
     __shared__ __attribute__((aligned(16))) float s_t[2][kSpT][HD + 4];
     __shared__ int s_e[2][kSpT];
@@ -1915,7 +1915,7 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
             const int e = sm_exp(mx), o = (kh * nt + tile) * kSpT + key;
             s_e[m][key] = m && bad ? kVBad : e;
             if (m) vexp[o] = bad ? kVBad : mx == 0.f ? -300 : 14 - e;   // a zero row has no weight
-            else kscale[o] = ldexpf(1.f, -e);
+            else kexp[o] = -e;
         }
     }
     __syncthreads();
@@ -1948,8 +1948,7 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
 struct AttnSplitArgs {
     const float *qn;       // [S][H][hd] normed, rotated
     const uint4 *planes;   // [KH][ntile][K units | V units]
-    const float *kscale;   // [KH][ntile 32]
-    const int *vexp;
+    const int *kexp, *vexp;   // [KH][ntile 32]
     float *part;           // [S][H][np][hd] context sums of a part, relative to its maximum
     float2 *ml;            // [S][H][np] (maximum, sum)
     int S, H, KH, pos_base, ntile, hw, chunk, np;   // hw: heads per block; chunk: key tiles per part
@@ -1961,8 +1960,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     constexpr int NS = HD / 16, ND = HD / 32, kU = KvPlanes<HD>::kUnits, kLd = 2 * kU / 256;
     constexpr int kRd = 3;   // operand reads run this many steps ahead of their products
     __shared__ uint4 s_kv0[2 * kU], s_kv1[2 * kU];
-    __shared__ __attribute__((aligned(16))) float s_ks0[kSpT], s_ks1[kSpT];
-    __shared__ __attribute__((aligned(16))) int s_ve0[kSpT], s_ve1[kSpT];
+    __shared__ __attribute__((aligned(16))) int s_ke0[kSpT], s_ke1[kSpT], s_ve0[kSpT], s_ve1[kSpT];
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, col = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // block -> part, row block (the longest first), head group
@@ -1978,7 +1976,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // a tile straight to LDS (no registers: the q operands and the context take 256 of them); the
     // two buffers are arrays of their own, so that the reads of one need not wait for the other's
     // copies
-    auto copy = [&](int t, uint4 *dst, float *ks, int *ve) {
+    auto copy = [&](int t, uint4 *dst, int *ke, int *ve) {
         typedef const __attribute__((address_space(1))) void *gp;
         typedef __attribute__((address_space(3))) void *lp;
 #pragma unroll
@@ -1986,13 +1984,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             __builtin_amdgcn_global_load_lds((gp)(src + (size_t)t * 2 * kU + tid + 256 * i), (lp)(dst + 256 * i + wave * 64),
                                              16, 0, 0);
         if (tid < kSpT) {
-            __builtin_amdgcn_global_load_lds((gp)(a.kscale + (kh * a.ntile + t) * kSpT + tid), (lp)ks, 4, 0, 0);
+            __builtin_amdgcn_global_load_lds((gp)(a.kexp + (kh * a.ntile + t) * kSpT + tid), (lp)ke, 4, 0, 0);
             __builtin_amdgcn_global_load_lds((gp)(a.vexp + (kh * a.ntile + t) * kSpT + tid), (lp)ve, 4, 0, 0);
         }
     };
     // the wave's query rows as B operands
     sm_h8 qh[NS], ql[NS];
-    float qs;
+    int qe;   // of the query row's power of two, as kexp
     {
         const float *qr = a.qn + ((size_t)sq * a.H + h) * HD + 8 * half;
         float mx = 0.f;
@@ -2002,7 +2000,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             for (int j = 0; j < 8; j++) mx = fmaxf(mx, fabsf(qr[16 * i + j]));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         const int e = sm_exp(mx);
-        qs = ldexpf(a.scale, -e);
+        qe = -e;
 #pragma unroll
         for (int i = 0; i < NS; i++) {
             float v[8];
@@ -2014,7 +2012,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             ql[i] = __builtin_bit_cast(sm_h8, lo);
         }
     }
-    copy(t0, s_kv0, s_ks0, s_ve0);
+    copy(t0, s_kv0, s_ke0, s_ve0);
     __builtin_amdgcn_s_waitcnt(kVm0);
     lds_barrier();
     sm_f16 acc[ND];
@@ -2024,11 +2022,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         for (int r = 0; r < 16; r++) acc[d][r] = 0.f;
     float m = -INFINITY, l = 0.f, A = 0.f;   // l: this lane's keys; A: the largest weight, R its exponent
     int R = 0;
-    auto tile = [&](int t, const uint4 *K, const float *ks, const int *ve, uint4 *next, float *nks, int *nve) {
+    auto tile = [&](int t, const uint4 *K, const int *ke, const int *ve, uint4 *next, int *nke, int *nve) {
         const int tn = min(t + 1, t1 - 1);   // the last tile is copied once more, into the free buffer
         const uint4 *V = K + kU;
         sm_f16 th;
-        copy(tn, next, nks, nve);   // their last reads are a barrier back
+        copy(tn, next, nke, nve);   // their last reads are a barrier back
         if (t <= wlast) {   // wave uniform
 #pragma unroll
             for (int r = 0; r < 16; r++) th[r] = 0.f;
@@ -2054,12 +2052,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             float pr[16], mx = -INFINITY;
 #pragma unroll
             for (int r4 = 0; r4 < 4; r4++) {
-                const float4 k4 = *(const float4 *)&ks[8 * r4 + 4 * half];
-                const float kk[4] = {k4.x, k4.y, k4.z, k4.w};
+                const int4 k4 = *(const int4 *)&ke[8 * r4 + 4 * half];
+                const int kk[4] = {k4.x, k4.y, k4.z, k4.w};
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const int r = 4 * r4 + i, kpos = t * kSpT + 8 * r4 + 4 * half + i;
-                    pr[r] = kpos <= qpos ? th[r] * (kk[i] * qs) : -INFINITY;
+                    // one power of two: those of a large key and a large query leave the range by themselves
+                    pr[r] = kpos <= qpos ? ldexpf(th[r] * a.scale, kk[i] + qe) : -INFINITY;
                     mx = fmaxf(mx, pr[r]);
                 }
             }
@@ -2125,8 +2124,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         lds_barrier();
     };
     for (int t = t0; t < t1; t += 2) {
-        tile(t, s_kv0, s_ks0, s_ve0, s_kv1, s_ks1, s_ve1);
-        if (t + 1 < t1) tile(t + 1, s_kv1, s_ks1, s_ve1, s_kv0, s_ks0, s_ve0);
+        tile(t, s_kv0, s_ke0, s_ve0, s_kv1, s_ke1, s_ve1);
+        if (t + 1 < t1) tile(t + 1, s_kv1, s_ke1, s_ve1, s_kv0, s_ke0, s_ve0);
     }
     if (s0 + col >= a.S) return;
     l += __shfl_xor(l, 32);
@@ -2303,7 +2302,7 @@ static bool put_vec(float **d, int *have, const float *h, int n, const char *who
 // ---------------------------------------------------------------- work buffers
 enum {
     W_Q, W_K, W_V, W_CTX, W_PART, W_QKV, W_Z, W_Y, W_AB, W_NRM, W_LOGIT, W_IDX, W_IO_X, W_IO_R, W_IO_P, W_IO_O,
-    W_HIST, W_BND, W_SQKV, W_SZ, W_SY, W_ROPE, W_GQN, W_GKN, W_GVV, W_GMAT, W_APL, W_AKS, W_AVE, W_APT, W_AML, W_COUNT
+    W_HIST, W_BND, W_SQKV, W_SZ, W_SY, W_ROPE, W_GQN, W_GKN, W_GVV, W_GMAT, W_APL, W_AKE, W_AVE, W_APT, W_AML, W_COUNT
 };
 struct WorkBuf {
     void *p = nullptr;
@@ -2998,16 +2997,16 @@ static bool attn_rows_split(const KvState &kv, const float *qn, const float *qra
     a.chunk = max((int)want, max(4, (a.ntile + 15) / 16));
     a.np = (a.ntile + a.chunk - 1) / a.chunk;
     uint4 *planes = (uint4 *)wbuf(W_APL, (size_t)d.KH * a.ntile * 2 * KvPlanes<HD>::kUnits * 4);
-    float *ks = wbuf(W_AKS, (size_t)d.KH * a.ntile * kSpT);
+    int *ke = (int *)wbuf(W_AKE, (size_t)d.KH * a.ntile * kSpT);
     int *ve = (int *)wbuf(W_AVE, (size_t)d.KH * a.ntile * kSpT);
     a.part = wbuf(W_APT, (size_t)S * d.H * a.np * HD);
     a.ml = (float2 *)wbuf(W_AML, (size_t)S * d.H * a.np * 2);
-    if (!planes || !ks || !ve || !a.part || !a.ml) return false;
+    if (!planes || !ke || !ve || !a.part || !a.ml) return false;
     a.qn = qn;
     a.planes = planes;
-    a.kscale = ks;
+    a.kexp = ke;
     a.vexp = ve;
-    hipLaunchKernelGGL(kv_split<HD>, dim3(a.ntile, d.KH), dim3(256), 0, st, kv.K, kv.V, d.max_t, nkeys, planes, ks, ve);
+    hipLaunchKernelGGL(kv_split<HD>, dim3(a.ntile, d.KH), dim3(256), 0, st, kv.K, kv.V, d.max_t, nkeys, planes, ke, ve);
     hipLaunchKernelGGL(attn_split<HD>, dim3((unsigned)((long)nhg * nrb * a.np)), dim3(256), 0, st, a);
     hipLaunchKernelGGL(attn_parts_merge<HD>, dim3(S, d.H), dim3(HD), 0, st, a, qraw, ctx);
     const hipError_t e = hipGetLastError();

@@ -274,6 +274,25 @@ def test_gqa_rows_v_scales(lib, lorc_omp, gen, zeros, exp):
         assert np.linalg.norm(y[s] - ref[s]) <= 1e-4 * np.linalg.norm(ref[s]), s
 
 
+def test_gqa_rows_qk_scales(lib, lorc_omp, gen):
+    """Queries of about 2^30 over cached keys of 2^-30, and one key of 2^127 in a dimension that
+    every query has as 0: its score is 0, though the powers of two of the two rows together
+    are past the fp32 range."""
+    dim = 20   # past the rotated ones
+
+    def scales(W):
+        W.q.sz.reshape(W.H, 2, W.hd, -1, 2)[:, 0, dim, :, 0] = 0.0
+        W.qn[:] = 2.0 ** 30
+        W.kn[:] = -1.0
+    Kc, Vc, run, oracle = _parts_block(lib, gen, 150, 7, scales)
+    Kc *= np.float32(2.0 ** -30)
+    Kc[:, 70] = 0.0
+    Kc[:, 70, dim] = 2.0 ** 127
+    y, ref = run(), oracle(lorc_omp)
+    for s in range(len(y)):
+        assert _util.maxrel_scaled(y[s], ref[s]) <= TOL, s
+
+
 # ---------------------------------------------------------------- GDN block
 host_params = _layers.gdn_host_params
 
