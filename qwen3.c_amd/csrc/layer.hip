@@ -1876,10 +1876,14 @@ __global__ __launch_bounds__(64) void qk_rows(const float *__restrict__ qraw, co
 // kernel 736.  Relative error of the layer against 64 bits 4.8e-7, before 1.1e-6.
 constexpr int kVm0 = 0x0F70;   // s_waitcnt vmcnt(0)
 constexpr int kSpT = 32;   // keys per tile, query rows per wave
-// Exponent of a V row with an infinity or NaN: its planes are zeros, and only the queries that
-// see the key give it a weight, an infinite one (so their context is NaN).  In the planes it
-// would reach the queries before it, whose weight 0 times it is NaN as well.
-constexpr int kVBad = 1 << 20;
+// Exponent of a K or V row with an infinity or NaN; its planes are zeros.
+//   V: only the queries that see the key give it a weight, an infinite one (so their context is
+//     NaN).  In the planes it would reach the queries before it, whose weight 0 times it is NaN
+//     as well.
+//   K: hi + lo of an infinity is NaN, where fp32 gives most queries an infinite score, and at
+//     -inf no weight.  The exponents of a tile with such a row are kBadTile larger, and its
+//     scores are summed in fp32.
+constexpr int kBad = 1 << 20, kBadTile = 1 << 22;
 template <int HD>
 struct KvPlanes {
     static constexpr int kUnits = HD / 16 * 2 * 64;   // 16-byte units of a tile's K; as many of V
@@ -1898,6 +1902,7 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
         *(float4 *)&s_t[m][key][4 * c4] = t < nkeys ? *(const float4 *)src : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     __syncthreads();
+    int kbad;
     {   // 4 threads per row
         const int m = tid >> 7, key = (tid >> 2) & 31, q = tid & 3;
         float mx = 0.f;
@@ -1912,19 +1917,24 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
         bad |= __shfl_xor(bad, 1);
         bad |= __shfl_xor(bad, 2);
         if (q == 0) {
-            const int e = sm_exp(mx), o = (kh * nt + tile) * kSpT + key;
-            s_e[m][key] = m && bad ? kVBad : e;
-            if (m) vexp[o] = bad ? kVBad : mx == 0.f ? -300 : 14 - e;   // a zero row has no weight
-            else kexp[o] = -e;
+            const int e = sm_exp(mx);
+            s_e[m][key] = bad ? kBad : e;
+            if (m) vexp[(kh * nt + tile) * kSpT + key] = bad ? kBad : mx == 0.f ? -300 : 14 - e;   // a zero row has no weight
         }
+        kbad = !m && bad;
     }
-    __syncthreads();
+    kbad = __syncthreads_or(kbad) ? kBadTile : 0;
+    if (tid < kSpT) {
+        const int e = s_e[0][tid];
+        kexp[(kh * nt + tile) * kSpT + tid] = (e == kBad ? kBad : -e) + kbad;
+    }
     uint4 *dst = planes + (size_t)(kh * nt + tile) * 2 * KvPlanes<HD>::kUnits;
     for (int i = tid; i < HD / 16 * 64; i += 256) {   // K: step i / 64, lane i % 64
         const int st = i >> 6, l = i & 63, key = l & 31;
         float v[8];
 #pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = ldexpf(s_t[0][key][16 * st + 8 * (l >> 5) + j], s_e[0][key]);
+        for (int j = 0; j < 8; j++)
+            v[j] = s_e[0][key] == kBad ? 0.f : ldexpf(s_t[0][key][16 * st + 8 * (l >> 5) + j], s_e[0][key]);
         uint4 hi, lo;
         sp_split8(v, hi, lo);
         dst[(2 * st) * 64 + l] = hi;
@@ -1936,7 +1946,7 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const int key = 16 * (u & 1) + 8 * (j >> 2) + 4 * (l >> 5) + (j & 3);
-            v[j] = s_e[1][key] == kVBad ? 0.f : ldexpf(s_t[1][key][d], s_e[1][key]);
+            v[j] = s_e[1][key] == kBad ? 0.f : ldexpf(s_t[1][key][d], s_e[1][key]);
         }
         uint4 hi, lo;
         sp_split8(v, hi, lo);
@@ -1947,11 +1957,12 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
 
 struct AttnSplitArgs {
     const float *qn;       // [S][H][hd] normed, rotated
+    const float *Kc;       // [KH][max_t][hd]
     const uint4 *planes;   // [KH][ntile][K units | V units]
     const int *kexp, *vexp;   // [KH][ntile 32]
     float *part;           // [S][H][np][hd] context sums of a part, relative to its maximum
     float2 *ml;            // [S][H][np] (maximum, sum)
-    int S, H, KH, pos_base, ntile, hw, chunk, np;   // hw: heads per block; chunk: key tiles per part
+    int S, H, KH, pos_base, max_t, ntile, hw, chunk, np;   // hw: heads per block; chunk: key tiles per part
     float scale;
 };
 
@@ -2050,6 +2061,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         }
         if (t <= wlast) {
             float pr[16], mx = -INFINITY;
+            const bool bad = __builtin_amdgcn_readfirstlane(ke[0]) >= kBadTile / 2;
+            const int se = bad ? qe - kBadTile : qe;
 #pragma unroll
             for (int r4 = 0; r4 < 4; r4++) {
                 const int4 k4 = *(const int4 *)&ke[8 * r4 + 4 * half];
@@ -2058,10 +2071,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                 for (int i = 0; i < 4; i++) {
                     const int r = 4 * r4 + i, kpos = t * kSpT + 8 * r4 + 4 * half + i;
                     // one power of two: those of a large key and a large query leave the range by themselves
-                    pr[r] = kpos <= qpos ? ldexpf(th[r] * a.scale, kk[i] + qe) : -INFINITY;
-                    mx = fmaxf(mx, pr[r]);
+                    pr[r] = kpos <= qpos ? ldexpf(th[r] * a.scale, kk[i] + se) : -INFINITY;
                 }
             }
+            if (bad) {   // wave uniform
+#pragma clang loop unroll(disable)
+                for (int key = 0; key < kSpT; key++) {
+                    if (__builtin_amdgcn_readfirstlane(ke[key]) != kBad + kBadTile) continue;
+                    const float *kr = a.Kc + ((size_t)kh * a.max_t + t * kSpT + key) * HD;
+                    const float *qr = a.qn + ((size_t)sq * a.H + h) * HD;
+                    float s = 0.f;
+#pragma clang loop unroll(disable)
+                    for (int d = 0; d < HD; d++) s += qr[d] * kr[d];
+                    s *= a.scale;
+                    if (s == -INFINITY && ve[key] == kBad) s = NAN;   // weight 0 of such a V row: not 0
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        if (8 * (r >> 2) + 4 * half + (r & 3) == key && t * kSpT + key <= qpos) pr[r] = s;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) mx = fmaxf(mx, pr[r]);
             mx = fmaxf(mx, __shfl_xor(mx, 32));
             const float mn = fmaxf(m, mx);
             const bool live = mn != -INFINITY;   // some key of the query seen so far
@@ -2076,7 +2106,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                     const int r = 4 * r4 + i;
                     const float e = pr[r] != -INFINITY ? expf(pr[r] - mn) : 0.f;   // NaN stays, also with no live key yet
                     ps += e;
-                    pr[r] = ee[i] == kVBad ? (pr[r] == -INFINITY ? 0.f : INFINITY) : ldexpf(e, ee[i]);
+                    pr[r] = ee[i] == kBad ? (pr[r] == -INFINITY ? 0.f : INFINITY) : ldexpf(e, ee[i]);
                     wm = fmaxf(wm, pr[r]);
                 }
             }
@@ -3003,6 +3033,8 @@ static bool attn_rows_split(const KvState &kv, const float *qn, const float *qra
     a.ml = (float2 *)wbuf(W_AML, (size_t)S * d.H * a.np * 2);
     if (!planes || !ke || !ve || !a.part || !a.ml) return false;
     a.qn = qn;
+    a.Kc = kv.K;
+    a.max_t = d.max_t;
     a.planes = planes;
     a.kexp = ke;
     a.vexp = ve;

@@ -247,6 +247,15 @@ def test_gqa_rows_cached_v_nonfinite(lib, gen, row, far, bad):
     assert not np.isfinite(y).any()
 
 
+def test_gqa_rows_cached_kv_nonfinite(lib, gen):
+    """A key whose score is -inf for some queries and whose V row is not finite: 0 times it is not
+    0, so every query is not finite (c/qwen.c:654-658)."""
+    Kc, Vc, run, _ = _parts_block(lib, gen, 150, 4)
+    Kc[0, 70, 40] = np.inf
+    Vc[0, 70, 3] = np.inf
+    assert not np.isfinite(run()).any()
+
+
 @pytest.mark.parametrize("r0,r1", [(3, 4), (0, 32), (0, 128), (128, 300)])
 def test_gqa_rows_cached_k_nan(lib, gen, r0, r1):
     """NaN K rows, whole tiles and parts of them: no query that sees one is finite."""
@@ -290,6 +299,23 @@ def test_gqa_rows_qk_scales(lib, lorc_omp, gen):
     Kc[:, 70, dim] = 2.0 ** 127
     y, ref = run(), oracle(lorc_omp)
     for s in range(len(y)):
+        assert _util.maxrel_scaled(y[s], ref[s]) <= TOL, s
+
+
+@pytest.mark.parametrize("dims", [(40,), (17, 63)])
+@pytest.mark.parametrize("row", [3, 200, 299])
+def test_gqa_rows_cached_k_inf(lib, lorc_omp, gen, row, dims):
+    """One cached K row with infinities: a query whose products with them are all -inf gives
+    the key no weight, the others are not finite (c/qwen.c:641-650), row by row as the
+    oracle's."""
+    Kc, Vc, run, oracle = _parts_block(lib, gen, 150, 2 + len(dims))
+    Kc[0, row, list(dims)] = np.inf
+    y, ref = run(), oracle(lorc_omp)
+    ok = np.isfinite(ref).all(axis=1)
+    assert ok.any() and not ok.all()
+    assert np.array_equal(np.isfinite(y).all(axis=1), ok)
+    assert not np.isfinite(y[~ok]).any()
+    for s in np.flatnonzero(ok):
         assert _util.maxrel_scaled(y[s], ref[s]) <= TOL, s
 
 
