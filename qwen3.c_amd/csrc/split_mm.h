@@ -132,7 +132,7 @@ struct SmLds {
     uint4 b[KW][2][NT * 32 * kSmUnits];
     float s[KW][2][2][RW * 32];    // scale
     float sz[KW][2][2][RW * 32];   // scale * (8 - zero)
-    float2 p[kSmMaxG][NT * 32];    // (p, sum) of the block's x rows
+    float2 p[kSmMaxG + 1][NT * 32];   // (p, sum) of the block's x rows; after the last group zeros
 };
 
 // What a wave and its threads bring.  wr / wo: weight descriptors and byte offsets of this
@@ -291,7 +291,7 @@ __device__ __forceinline__ void sm_product(SmLds<RW, KW, NT> &L, const SmSrc<RW,
         };
 #pragma unroll
         for (int f = 0; f < kAhead; f++) b_read(f);
-        float pn = L.p[min(g, src.ng - 1)][xrow].x;
+        float pn = L.p[min(g, src.ng)][xrow].x;
         const float az = h ? L.sz[kw][sbuf][half][rw * 32 + xrow] : 0.f;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -318,7 +318,7 @@ __device__ __forceinline__ void sm_product(SmLds<RW, KW, NT> &L, const SmSrc<RW,
             if (tt == 0 && (k & 3) == 3) fs[k >> 2] = *(const float4 *)&L.s[kw][sbuf][h][rw * 32 + 8 * (k >> 2) + 4 * half];
             if (k == 15) {
                 fp = pn;
-                if (tt + 1 < NT) pn = L.p[min(g, src.ng - 1)][(tt + 1) * 32 + xrow].x;
+                if (tt + 1 < NT) pn = L.p[min(g, src.ng)][(tt + 1) * 32 + xrow].x;
             }
             // the zero points of the pair: acc += (s (8 - z)) xsum, one fp32 product of K = 2 groups
             // (lane: row or column l % 32, group l / 32 of the pair)
@@ -337,10 +337,12 @@ __device__ __forceinline__ void sm_product(SmLds<RW, KW, NT> &L, const SmSrc<RW,
 #pragma unroll
     for (int k = 0; k < kXV; k++) x_load(2 * s0 + 1, k, xv[1]);
     // (p, sum) of every group of the block's x rows: read by each wave from global memory they
-    // took as long as the x planes (one 8-byte word of 32 rows per load)
-    for (int g = 2 * wave + half; g < src.ng; g += 2 * RW * KW)
+    // took as long as the x planes (one 8-byte word of 32 rows per load).  The half pair past an odd
+    // count has the next row's codes, whose sums may be past the fp32 range: power 0, not scale
+    // 0 alone, which times infinity is NaN
+    for (int g = 2 * wave + half; g <= src.ng; g += 2 * RW * KW)
 #pragma unroll
-        for (int i = 0; i < NT; i++) L.p[g][i * 32 + xrow] = src.xp[i][g];
+        for (int i = 0; i < NT; i++) L.p[g][i * 32 + xrow] = g < src.ng ? src.xp[i][g] : make_float2(0.f, 0.f);
 #pragma unroll
     for (int k = 0; k < kXV; k++) x_store(0, k, xv[0]);
     s_store(0, s0, sv);

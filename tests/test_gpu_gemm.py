@@ -118,6 +118,18 @@ def test_gemm_split_limits(lib, gen):
     assert np.max(np.abs(y[1] - y64[1])) <= 8 * 2.0 ** -149 * (I // gs)
 
 
+@pytest.mark.parametrize("O,I,S", [(34, 384, 8), (100, 1152, 8), (4098, 1152, 97), (2560, 1152, 640), (6100, 896, 130)])
+def test_gemm_split_odd_groups_limits(lib, O, I, S):
+    """Odd group counts and x whose sums with every second row's codes (n - 8 = 7) pass the fp32
+    range: the rows between them (n - 8 = 1) are exact, though the half pair past their last
+    group holds the next row's codes."""
+    q = np.repeat(np.tile(np.array([0x99, 0xFF], np.uint8), O // 2), I // 2)
+    sz = np.tile(np.array([2.0 ** -10, 8.0], np.float32), O * I // 128)
+    y = lib.matmul(lib.tensor(q, sz, 6, I, O, 128), np.full(S * I, 2.0 ** 120, np.float32), S=S).reshape(S, O)
+    assert np.all(y[:, 0::2] == I * np.float32(2.0 ** 110))
+    assert not np.isfinite(y[:, 1::2]).any()
+
+
 def test_gemm_wide_range_rows(lib, orc_omp, gen):
     """Rows of x whose groups span many binades (each group scaled by 2^k, k in -20..20):
     the per-(row, group) exponent of the digit decomposition follows each group."""
