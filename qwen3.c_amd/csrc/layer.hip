@@ -2332,7 +2332,7 @@ static bool put_vec(float **d, int *have, const float *h, int n, const char *who
 // ---------------------------------------------------------------- work buffers
 enum {
     W_Q, W_K, W_V, W_CTX, W_PART, W_QKV, W_Z, W_Y, W_AB, W_NRM, W_LOGIT, W_IDX, W_IO_X, W_IO_R, W_IO_P, W_IO_O,
-    W_HIST, W_BND, W_SQKV, W_SZ, W_SY, W_ROPE, W_GQN, W_GKN, W_GVV, W_GMAT, W_APL, W_AKE, W_AVE, W_APT, W_AML, W_COUNT
+    W_HIST, W_BND, W_SQKV, W_SZ, W_SY, W_ROPE, W_GQN, W_GKN, W_GVV, W_GMAT, W_APL, W_APT, W_COUNT
 };
 struct WorkBuf {
     void *p = nullptr;
@@ -3026,12 +3026,21 @@ static bool attn_rows_split(const KvState &kv, const float *qn, const float *qra
     const long want = (steps * nhg + 2 * n_cu() - 1) / (2 * n_cu());
     a.chunk = max((int)want, max(4, (a.ntile + 15) / 16));
     a.np = (a.ntile + a.chunk - 1) / a.chunk;
-    uint4 *planes = (uint4 *)wbuf(W_APL, (size_t)d.KH * a.ntile * 2 * KvPlanes<HD>::kUnits * 4);
-    int *ke = (int *)wbuf(W_AKE, (size_t)d.KH * a.ntile * kSpT);
-    int *ve = (int *)wbuf(W_AVE, (size_t)d.KH * a.ntile * kSpT);
-    a.part = wbuf(W_APT, (size_t)S * d.H * a.np * HD);
-    a.ml = (float2 *)wbuf(W_AML, (size_t)S * d.H * a.np * 2);
-    if (!planes || !ke || !ve || !a.part || !a.ml) return false;
+    // The scratch does not grow with the position from one piece of a prompt to the next (a growth
+    // waits for the stream, frees and allocates: 0.4 ms a call): key planes and exponents for
+    // 4096 keys, then for doubled counts, at most the cache's; the parts for the most that S rows
+    // have at any position (n row blocks hold at least n ntile / 2 key tiles).
+    const int tmax = (d.max_t + kSpT - 1) / kSpT;
+    size_t tcap = 4096 / kSpT;
+    while (tcap < (size_t)a.ntile) tcap *= 2;
+    tcap = d.KH * (size_t)max(a.ntile, (int)min(tcap, (size_t)tmax));
+    const int pcap = max(a.np, min(min(16, 4 * n_cu() / (nrb * nhg) + 1), (tmax + 3) / 4));
+    const size_t rows_h = (size_t)S * d.H * pcap;
+    uint4 *planes = (uint4 *)wbuf(W_APL, tcap * (2 * KvPlanes<HD>::kUnits * 4 + 2 * kSpT));
+    a.part = wbuf(W_APT, rows_h * (HD + 2));
+    if (!planes || !a.part) return false;
+    int *ke = (int *)(planes + tcap * 2 * KvPlanes<HD>::kUnits), *ve = ke + tcap * kSpT;
+    a.ml = (float2 *)(a.part + rows_h * HD);
     a.qn = qn;
     a.Kc = kv.K;
     a.max_t = d.max_t;

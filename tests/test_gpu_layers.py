@@ -319,6 +319,23 @@ def test_gqa_rows_cached_k_inf(lib, lorc_omp, gen, row, dims):
         assert _util.maxrel_scaled(y[s], ref[s]) <= TOL, s
 
 
+def test_gqa_rows_pieces_scratch(lib, gen):
+    """A prompt in pieces of one size up to position 8192: the scratch that a position needs is
+    taken when it doubles, not piece by piece (a growth waits for the device)."""
+    import torch
+    D, H, KH, hd, rot, max_t, S = 256, 4, 2, 256, 64, 8192, 256
+    W = _layers.GqaWeights(gen, gen.stream(0x9FD0, 1), D, H, KH, hd, rot, 128)
+    t = [m.upload(lib) for m in (W.q, W.k, W.v, W.o)]
+    lib.kv_ensure(151, KH * max_t, hd, hd)
+    lib.gqa_norm_weight(151, W.qn, W.kn)
+    xs = gen.normal(S * D, 0x9FD1)
+    free = []
+    for pos in range(0, max_t, S):
+        lib.gqa_full(151, xs, *t, S, H, KH, hd, rot, pos, max_t, W.eps, W.theta)
+        free.append(torch.cuda.mem_get_info()[0])
+    assert sum(a != b for a, b in zip(free, free[1:])) <= 1, free
+
+
 # ---------------------------------------------------------------- GDN block
 host_params = _layers.gdn_host_params
 
