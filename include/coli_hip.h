@@ -296,6 +296,10 @@ int   coli_hip_eg_force_gemv(int force_gemv);
  * the decode block (0); returns the previous setting.  A test and bench hook with no
  * counterpart in the reference. */
 int   coli_hip_gqa_seq(int on);
+/* The tile that the dense GEMM takes for S rows of x: output rows of a block (256, 128 or 64;
+ * 0 when these rows take another path) and, in *parts, the parts that the block's waves split
+ * the groups into.  A test hook with no counterpart in the reference. */
+int   coli_hip_gemm_tile(const ColiVkTensor *t, int S, int *parts);
 /* coli_vk_gdn_full_seq's recurrence in closed form per 64-token chunk (1, the default) or
  * token by token (0); returns the previous setting.  A test and bench hook with no
  * counterpart in the reference. */

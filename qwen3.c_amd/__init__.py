@@ -77,6 +77,7 @@ _SIGS = {
     "coli_hip_moe_cert_all": (_I, [_I]),
     "coli_hip_eg_force_gemv": (_I, [_I]),
     "coli_hip_gqa_seq": (_I, [_I]),
+    "coli_hip_gemm_tile": (_I, [_P, _I, C.POINTER(_I)]),
     "coli_hip_gdn_chunked": (_I, [_I]),
     "coli_hip_st_open": (_P, [C.c_char_p]),
     "coli_hip_st_close": (None, [_P]),
@@ -435,6 +436,12 @@ class Lib:
         """coli_vk_gqa_full over S >= 4 rows batched (True) or token by token (False);
         returns the previous setting."""
         return bool(self.L.coli_hip_gqa_seq(1 if on else 0))
+
+    def gemm_tile(self, t, S):
+        """The dense GEMM's tile for S rows of x: (output rows of a block, parts of the groups),
+        (0, 0) when they take another path."""
+        parts = _I(0)
+        return int(self.L.coli_hip_gemm_tile(t.handle, S, C.byref(parts))), parts.value
 
     def gdn_chunked(self, on):
         """coli_vk_gdn_full_seq's recurrence per 64-token chunk (True) or token by token;

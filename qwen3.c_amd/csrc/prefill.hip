@@ -1133,32 +1133,36 @@ bool gemm6_ok(const ColiVkTensor *t) {
 }
 
 template <int RW, int KW, int NT>
-static bool gemm6_launch(GemmArgs &g, int min_blocks, hipStream_t st) {
+static void gemm6_launch(GemmArgs &g, hipStream_t st) {
     g.nu = (g.O + RW * 32 - 1) / (RW * 32);
     g.npass = (g.S + NT * 32 - 1) / (NT * 32);
-    if ((long)g.nu * g.npass < min_blocks) return false;
     hipLaunchKernelGGL((gemm6_split<RW, KW, NT>), dim3(8 * ((g.nu + 7) / 8) * g.npass), dim3(RW * KW * 64), 0, st, g);
-    return true;
 }
 
 // The largest tile that still gives most CUs a block: 256 rows x 64 of x moves the fewest x
 // planes; fewer rows and 32 of x fill the chip sooner, with the groups split over the block's
-// waves where there are enough of them.  us per call, digits included (O x I x S; tiles 256 x 64,
+// waves where there are enough of them.  us per call, the split of x included (O x I x S; tiles 256 x 64,
 // 128 x 32 unsplit, 128 x 32 in 2 parts, 64 x 32 in 2, 64 x 32 in 4; the int8 kernel before):
 //   8192 x 2048 x 512: 49.9, 58.5, 68.2, 69.8, 93.5; 56.2   4096 x 2048 x 777: 45.2, 55.0, 67, 64, 86; 57.2
 //   2048 x 4096 x 512: 62.6, 36.9, 34.4, 38.9, 45.0; 43.5   12288 x 512 x 100: 16.1, 12.6, 15.0, 13.4, 22.2; 13.1
 //    512 x 2048 x 512: 38.5, 22.9, 21.1, 17.9, 18.2; 26.0    2048 x 4096 x 45: 56.4, 30.2, 25.7, 20.6, 19.1; 36.9
 //   8192 x 2048 x  45: 33.1, 18.7, 16.7, 14.4, 14.7; 21.8    2048 x 4096 x  8: 51.9, 28.5, 23.8, 19.1, 17.3; 25.4
+struct GemmTile {
+    int rows, parts;   // output rows of a block, parts of its groups; 64 rows of x with 256, else 32
+};
+static GemmTile gemm6_tile(int O, int I, int S) {
+    const auto blocks = [&](int rows, int xrows) { return (long)((O + rows - 1) / rows) * ((S + xrows - 1) / xrows); };
+    const int cu = n_cu(), parts = I / kGS <= 8 ? 1 : 2;
+    if (blocks(256, 64) >= cu * 5 / 8) return {256, 1};
+    if (blocks(128, 32) >= cu * 3 / 4) return {128, parts};
+    return {64, 2 * parts};
+}
+
 static void gemm6_dispatch(GemmArgs &g, hipStream_t st) {
-    const int cu = n_cu(), ng = g.I / kGS;
-    if (gemm6_launch<8, 1, 2>(g, cu * 5 / 8, st)) return;
-    if (ng <= 8) {
-        if (gemm6_launch<4, 1, 1>(g, cu * 3 / 4, st)) return;
-        gemm6_launch<2, 2, 1>(g, 0, st);
-    } else {
-        if (gemm6_launch<4, 2, 1>(g, cu * 3 / 4, st)) return;
-        gemm6_launch<2, 4, 1>(g, 0, st);
-    }
+    const GemmTile t = gemm6_tile(g.O, g.I, g.S);
+    if (t.rows == 256) gemm6_launch<8, 1, 2>(g, st);
+    else if (t.rows == 128) t.parts == 1 ? gemm6_launch<4, 1, 1>(g, st) : gemm6_launch<4, 2, 1>(g, st);
+    else t.parts == 2 ? gemm6_launch<2, 2, 1>(g, st) : gemm6_launch<2, 4, 1>(g, st);
 }
 
 bool gemm6(const ColiVkTensor *const *t, float *const *d_y, int nt, const float *d_x, int S, hipStream_t st,
@@ -1312,6 +1316,13 @@ void prefill_shutdown() {
 }  // namespace coli
 
 using namespace coli;
+
+COLI_API int coli_hip_gemm_tile(const ColiVkTensor *t, int S, int *parts) {
+    if (!ok() || !gemm6_ok(t) || S < kGemmMinS) return 0;
+    const GemmTile tile = gemm6_tile(t->O, t->I, S);
+    if (parts) *parts = tile.parts;
+    return tile.rows;
+}
 
 // The layer's MoE block over S token rows d_xs [S, D] (prefill), expert projections on
 // MFMA: d_out [S, D]; d_idx / d_val [S, K] (routing, rank order) may be NULL.

@@ -72,19 +72,25 @@ def test_gemm_rows(lib, orc_omp, gen, O, I, S):
     _check(y, q, sz, x, S, I, O, gs, yo, f"gemm O={O} I={I} S={S}")
 
 
-@pytest.mark.parametrize("O,I,S", [(4, 128, 4), (100, 128, 31), (65, 384, 33), (2049, 1024, 97), (31, 1152, 64),
-                                   (6200, 1152, 130), (4100, 128, 641), (5121, 640, 515), (2560, 2176, 520)])
-def test_gemm_split_tiles(lib, gen, O, I, S):
-    """Every tile of the dense GEMM (256 x 64, 128 x 32, 64 x 32; whole, in 2 and in 4 parts of
-    the groups) at row counts just past and short of a tile, one group, odd group counts and
-    parts without a group, against the f64 product.  Per output the error is at most that of
+@pytest.mark.parametrize("O,I,S,tile", [
+    (4, 128, 4, (64, 2)), (100, 128, 31, (64, 2)), (65, 384, 33, (64, 2)), (2049, 1024, 97, (64, 2)),
+    (31, 1152, 64, (64, 4)), (1025, 1280, 65, (64, 4)), (12288, 512, 100, (128, 1)), (4097, 1024, 193, (128, 1)),
+    (6100, 896, 130, (128, 1)), (6200, 1152, 130, (128, 2)), (2560, 2176, 520, (128, 2)), (4100, 128, 641, (256, 1)),
+    (5121, 640, 515, (256, 1))])
+def test_gemm_split_tiles(lib, gen, O, I, S, tile):
+    """Every tile of the dense GEMM (256 x 64, 128 x 32 whole and in 2 parts of the groups,
+    64 x 32 in 2 and in 4; the library names the one it takes) at row counts just past and
+    short of a tile, one group, odd group counts and parts without a group, against the f64
+    product.  Per output the error is at most that of
     the x planes (2^-23 of each x) and of the fp32 sums (16 steps in a group, then one per
     group and part, each 2^-24 of the partial sum, and the scale's and zero's roundings), all
     of them relative to sum |s| (|n - 8| + |z - 8|) |x|."""
     gs = 128
     q, sz = gen.fmt6(O, I, gs, 0x6E30 + O)
     x = gen.normal(S * I, 0x6E31 + I)
-    y = lib.matmul(lib.tensor(q, sz, 6, I, O, gs), x, S=S).reshape(S, O)
+    t = lib.tensor(q, sz, 6, I, O, gs)
+    assert lib.gemm_tile(t, S) == tile
+    y = lib.matmul(t, x, S=S).reshape(S, O)
     y64 = _f64_rows(q, sz, x, S, I, O, gs)
     b = q.reshape(O, I // 2)
     nib = np.empty((O, I), np.float64)
@@ -97,8 +103,9 @@ def test_gemm_split_tiles(lib, gen, O, I, S):
 
 
 def test_gemm_split_limits(lib, gen):
-    """Rows at the ends of the fp32 range: all zero, subnormal, near the largest number, and one
-    group 2^60 above the others; each row relative to its own product."""
+    """Rows towards the ends of the fp32 range: all zero, subnormal, 2^110 (a group's sum of x and
+    its products with n - 8 have to stay below 2^128: any |x| < 2^117 does), and one group 2^60
+    above the others; each row relative to its own product."""
     O, I, gs = 96, 512, 128
     q, sz = gen.fmt6(O, I, gs, 0x6E40)
     x = gen.normal(8 * I, 0x6E41).reshape(8, I)
@@ -132,7 +139,7 @@ def test_gemm_split_odd_groups_limits(lib, O, I, S):
 
 def test_gemm_wide_range_rows(lib, orc_omp, gen):
     """Rows of x whose groups span many binades (each group scaled by 2^k, k in -20..20):
-    the per-(row, group) exponent of the digit decomposition follows each group."""
+    the exponent of each row and group's split follows the group."""
     O, I, S, gs = 512, 2048, 12, 128
     q, sz = gen.fmt6(O, I, gs, 0x6E10)
     x = gen.normal(S * I, 0x6E11).reshape(S, I // gs, gs)
@@ -146,7 +153,7 @@ def test_gemm_wide_range_rows(lib, orc_omp, gen):
 
 
 def test_gemm_pair_rows(lib, orc_omp, gen):
-    """matmul_pair at S = 40: one digit decomposition of x serves both tensors."""
+    """matmul_pair at S = 40: one split of x serves both tensors."""
     I, gs, S = 2048, 128, 40
     q1, s1 = gen.fmt6(512, I, gs, 0x6E20)
     q2, s2 = gen.fmt6(1000, I, gs, 0x6E21)
