@@ -168,8 +168,10 @@ def test_rows_f01(lib, orc, gen, fmt, O, I, S):
 @pytest.mark.parametrize("fmt,O,I,S", [(0, 256, 132, 768), (0, 257, 260, 737), (1, 1000, 388, 197), (0, 33, 4, 4090),
                                          (1, 1000, 388, 262), (1, 257, 36, 993)])
 def test_rows_f01_many(lib, orc, gen, fmt, O, I, S):
-    """Rows enough for the kernel with its products on the matrix cores: the same bits as the
-    sequential sums, also where the products are subnormal, zero of either sign or huge."""
+    """Rows enough for the kernel with its products on the matrix cores (from three 16 x 16 tiles
+    per CU, int8 from four; the int8 case of 197 rows lies below that and takes the other one):
+    the same bits as the sequential sums, also where the products are subnormal, zero of
+    either sign or huge."""
     x = gen.normal(S * I, 0x3110 + S).reshape(S, I)
     x[1] *= np.float32(2.0 ** -126)
     x[2] *= np.float32(2.0 ** -138)

@@ -182,7 +182,8 @@ def test_gqa_row_tiles(lib, lorc_omp, gen, shape, spread):
 def test_gqa_rows_nonfinite(lib, gen, row, bad):
     """One row of x with a NaN or an infinity: the rows before it see none of it, also those
     of its 32-row and 32-key tile (the same bits as with a finite row there), the rows from it
-    on are not finite (its key and value are in their sums, c/qwen.c:641-660)."""
+    on are not finite (its key and value are in their sums, c/qwen.c:641-660; rows whose value
+    alone is not finite: test_gqa_rows_cached_v_nonfinite)."""
     D, H, KH, hd, rot, max_t, layer, S, pos = 256, 4, 2, 64, 16, 100, 50, 65, 0
     W = _layers.GqaWeights(gen, gen.stream(0x9F70, layer), D, H, KH, hd, rot, 128)
     tq, tk, tv, to = (m.upload(lib) for m in (W.q, W.k, W.v, W.o))

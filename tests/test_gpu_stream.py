@@ -268,3 +268,34 @@ def test_stream_rows_ab_cfg3(lib, lorc, gen, moe_cfg, ab_fmt):
                          state_base=115 + 2 * ab_fmt)
     _run_stream(lib, lorc, stack, L.router, 8, 2, True, 0xE680 + ab_fmt, gen)
     assert lib.moe_error() == 0
+
+
+@pytest.mark.parametrize("ab_fmt", [0, 1])
+@pytest.mark.parametrize("D", [2176, 3968, 4096])
+def test_stream_rows_ab_wide(lib, lorc, gen, D, ab_fmt):
+    """f32 and int8 a/b rows of more than 2048 columns (a second word per thread of the
+    recurrence launch, for some or for all of its threads): the recurrent state, which decay and
+    beta make, after each of three tokens, within 1e-4 of its largest value (128 columns left
+    out change a dot by a quarter of its deviation)."""
+    L = Layer(lib, gen, 0xE700 + D, D, 128, 16, 128)
+    import _moe
+    _moe._active[0] = None
+    first, K = 70, 4
+    lib.eg_table_init(first + 1, L.E, L.D, L.I, L.gs)
+    L.register(lib, first)
+    gqa = dict(H=4, KH=2, hd=64, rot=16, gs=128)
+    gdn = dict(KH=2, KD=64, VH=4, VD=32, K=4, gs=128)
+    stack = _stack.Stack(lib, gen, 0xE720 + D + ab_fmt, 1, D, gqa, gdn, L, max_t=16, ab_fmt=ab_fmt, first_layer=first,
+                         state_base=154)
+    G = stack.layers[0]
+    W = G["W"]
+    for t in range(3):
+        x = gen.normal(D, 0xE780 + D + ab_fmt + t)
+        lib.stream_begin(x)
+        stack.pipe_layer(lib, 0, t, K, L.router)
+        stack.oracle_layer(lorc, 0, x, t, K)
+        lib.stream_end(D)
+        ring, S = lib.gdn_state_read(G["idx"], W.K, W.CD, W.VH, W.KD, W.VD)
+        for got, ref in ((ring, G["state"][0]), (S, G["state"][1])):
+            assert np.max(np.abs(got.ravel() - ref)) <= 1e-4 * np.max(np.abs(ref)), t
+    assert lib.moe_error() == 0
