@@ -1894,15 +1894,15 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
                                                 int nkeys, uint4 *__restrict__ planes, int *__restrict__ kexp,
                                                 int *__restrict__ vexp) {
     __shared__ __attribute__((aligned(16))) float s_t[2][kSpT][HD + 4];
-    __shared__ int s_e[2][kSpT];
+    __shared__ int s_e[2][kSpT], s_k[kSpT], s_bad;
     const int tile = blockIdx.x, kh = blockIdx.y, nt = gridDim.x, tid = threadIdx.x;
+    if (tid == 0) s_bad = 0;
     for (int i = tid; i < 2 * kSpT * (HD / 4); i += 256) {
         const int m = i / (kSpT * (HD / 4)), key = i / (HD / 4) % kSpT, c4 = i % (HD / 4), t = tile * kSpT + key;
         const float *src = (m ? Vc : Kc) + ((size_t)kh * max_t + t) * HD + 4 * c4;
         *(float4 *)&s_t[m][key][4 * c4] = t < nkeys ? *(const float4 *)src : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     __syncthreads();
-    int kbad;
     {   // 4 threads per row
         const int m = tid >> 7, key = (tid >> 2) & 31, q = tid & 3;
         float mx = 0.f;
@@ -1916,25 +1916,24 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
         mx = fmaxf(mx, __shfl_xor(mx, 2));
         bad |= __shfl_xor(bad, 1);
         bad |= __shfl_xor(bad, 2);
+        if (bad)
+            for (int d = q; d < HD; d += 4) s_t[m][key][d] = 0.f;
         if (q == 0) {
             const int e = sm_exp(mx);
-            s_e[m][key] = bad ? kBad : e;
+            s_e[m][key] = e;
             if (m) vexp[(kh * nt + tile) * kSpT + key] = bad ? kBad : mx == 0.f ? -300 : 14 - e;   // a zero row has no weight
+            else s_k[key] = bad ? kBad : -e;
+            if (!m && bad) s_bad = kBadTile;
         }
-        kbad = !m && bad;
     }
-    kbad = __syncthreads_or(kbad) ? kBadTile : 0;
-    if (tid < kSpT) {
-        const int e = s_e[0][tid];
-        kexp[(kh * nt + tile) * kSpT + tid] = (e == kBad ? kBad : -e) + kbad;
-    }
+    __syncthreads();
+    if (tid < kSpT) kexp[(kh * nt + tile) * kSpT + tid] = s_k[tid] + s_bad;
     uint4 *dst = planes + (size_t)(kh * nt + tile) * 2 * KvPlanes<HD>::kUnits;
     for (int i = tid; i < HD / 16 * 64; i += 256) {   // K: step i / 64, lane i % 64
         const int st = i >> 6, l = i & 63, key = l & 31;
         float v[8];
 #pragma unroll
-        for (int j = 0; j < 8; j++)
-            v[j] = s_e[0][key] == kBad ? 0.f : ldexpf(s_t[0][key][16 * st + 8 * (l >> 5) + j], s_e[0][key]);
+        for (int j = 0; j < 8; j++) v[j] = ldexpf(s_t[0][key][16 * st + 8 * (l >> 5) + j], s_e[0][key]);
         uint4 hi, lo;
         sp_split8(v, hi, lo);
         dst[(2 * st) * 64 + l] = hi;
@@ -1946,7 +1945,7 @@ __global__ __launch_bounds__(256) void kv_split(const float *__restrict__ Kc, co
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const int key = 16 * (u & 1) + 8 * (j >> 2) + 4 * (l >> 5) + (j & 3);
-            v[j] = s_e[1][key] == kBad ? 0.f : ldexpf(s_t[1][key][d], s_e[1][key]);
+            v[j] = ldexpf(s_t[1][key][d], s_e[1][key]);
         }
         uint4 hi, lo;
         sp_split8(v, hi, lo);
