@@ -662,8 +662,11 @@ static int launch_lanes_mode(const ColiVkTensor *t, const float *x, float *y, hi
 }
 
 // S rows of x.  Lanes layout: one launch for up to kGemvRows of them, a set of blocks per
-// row.  The blocks of a row range sit on one XCD for every row (whole sets of 8), so its
-// weights come from HBM once: 4.4 us for two rows at 8192 x 2048, 8.0 with a launch per row.
+// row.  4.4 us for two rows at 8192 x 2048, 8.0 with a launch per row.  There a row has 256 blocks,
+// a whole number per XCD (workgroups go to the 8 XCDs round-robin), so a weight range is on one
+// XCD for both rows and comes from HBM once.  Counts that 8 does not divide put the rows' blocks of
+// a range on different XCDs, and each fetches it (5000 x 2048, 157 blocks: two rows take 1.35 to
+// 1.41 times one, 8192 x 2048 1.33 in the same run; with a launch per row 1.9).
 constexpr int kGemvRows = 16;
 static bool launch_rows(const ColiVkTensor *t, const float *x, float *y, int S, hipStream_t st) {
     if (t->layout == kLayoutLanes) {

@@ -121,7 +121,7 @@ bool argmax_decode_host(const unsigned long long *keys, uint32_t epoch, int *idx
 // fmt6 tensors of group size 128 sharing I (one split of x serves all).  gx:
 // x is the GatedDeltaNet recurrence output and goes through its gated output norm first.
 constexpr int kGemmMaxI = kLaneMaxI;
-constexpr int kGemmMinS = 4;            // fewer rows of x: one GEMV launch per row
+constexpr int kGemmMinS = 4;            // fewer rows of x: the GEMV, a set of blocks per row
 struct GatedX {
     const float *z;        // [S][I] z projection rows
     const float *gnorm;    // norm weight [VD] of row s at gnorm + s * gstride
