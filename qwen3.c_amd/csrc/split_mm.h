@@ -18,8 +18,9 @@
 //
 // What bounds it: on random data these products take 21 ns per SIMD with the whole chip busy
 // (15 with an eighth of it: the clock falls under the load), 26 ns with an LDS read and four
-// vector instructions each.  512 x 8192 x 2048 takes 43 us, 42 ns a product: the waves of a
-// block wait for each other once per group, and x staging takes the rest.
+// vector instructions each.  512 x 8192 x 2048 takes 43 us, 42 ns a product, the matrix cores
+// busy 34% of the time: the waves of a block wait for each other once per group (30% of their
+// cycles) and stand ready behind each other's reads and vector instructions (42%).
 //
 // Operands (v_mfma_f32_32x32x16_f16: lane l holds row / column l % 32 and 8 of 16 k in half
 // l / 32; the result's register r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4, column
@@ -168,7 +169,9 @@ __device__ __forceinline__ int sm_stage_row(int k) {
 // reads then fall on different banks
 __device__ __forceinline__ int sm_swz(int r) { return (r ^ ((r >> 3) & 3)) & 7; }
 
-// A operand of the 8 columns of one word (see above)
+// A operand of the 8 columns of one word (see above): the codes go into the mantissa of f16 1024 or
+// 1024 + 16 n, and the offset is subtracted (the conversion of Kim et al., "Who Says Elephants Can't
+// Run", 2022, here with codes stored XOR 8)
 __device__ __forceinline__ sm_h8 sm_a8(uint32_t w) {
     const uint32_t v = w >> 8;
     union {
